@@ -129,7 +129,9 @@ typedef struct kx_plan {
     int32_t gtiles; /* neighbouring image tiles per wave in the adjoint (1, 2
                        or 4; they share the staged trace windows),
                        0 = automatic */
-    int32_t pad0;
+    int32_t slots;  /* 1: every receiver table (off_r and, when dynamic, wp_r
+                       and wq_r) is followed in memory by its slot-ordered
+                       copy (kx_slot_table); 0: it is not */
     double wtyp;  /* typical |weight| of one (point, trace) pair: 1 kinematic,
                      mean_s |(wp_s, wq_s)| * mean_r |(wp_r, wq_r)| over the
                      nonzero weights dynamic (0: taken as wamp).  A float32
@@ -163,6 +165,16 @@ int kx_encode_table(const kx_plan *geom, const double *tabT, int32_t n,
  * (KX_F32, KX_F64 or KX_F16), zero padded (dynamic weights). */
 int kx_tile_table(const kx_plan *geom, const double *tabT, int32_t n,
                   int32_t fmt, void *out, void *stream);
+
+/* Slot-ordered copy of one receiver table in the tiled layout, written right
+ * behind it: tab holds ntiles*n*64 elements of fmt (KX_F32 or KX_F16; offsets
+ * or weights) and room for kx_slot_table_elems(geom, n) more.  The copy is
+ * the order in which the forward's blocks of 8 and 16 receivers read the
+ * table (plan.slots = 1): per tile and block of 16 receivers, chunks of 16
+ * bytes of consecutive points of one receiver, so that the lanes of a wave
+ * read contiguous memory.  (No reference counterpart: device layout.) */
+int64_t kx_slot_table_elems(const kx_plan *geom, int32_t n);
+int kx_slot_table(const kx_plan *geom, int32_t n, int32_t fmt, void *tab, void *stream);
 
 /* The engine kernels alone.
  * kx_spread: traces[ns*nr][nt] = sum over image points of m spread at the
@@ -218,6 +230,16 @@ int kx_xcorr_rows(const void *a, int64_t astride, int32_t la, const void *b, int
  * convolves them in LDS in the same launch (the data are bitwise those of
  * kx_spread followed by kx_conv) and leaves work untouched. */
 int kx_forward(const kx_plan *p, const void *m, void *d, void *work, void *stream);
+
+/* kx_forward with a workspace of work_bytes >= kx_workspace_bytes(p): a
+ * float32 forward whose receiver blocks do not fill the chip evenly then
+ * shares the image tiles of a block between several workgroups, each keeping
+ * its 64-bit sums in the workspace, and adds them in a second launch (the
+ * data are bitwise the same).  kx_forward_work_bytes() is the size with which
+ * it runs fastest; kx_forward passes kx_workspace_bytes(p). */
+int64_t kx_forward_work_bytes(const kx_plan *p);
+int kx_forward_ws(const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes,
+                  void *stream);
 int kx_adjoint(const kx_plan *p, const void *d, void *m, void *work, void *stream);
 
 /* kx_forward with no caller memory beyond m and d, for callers that cannot

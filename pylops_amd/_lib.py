@@ -22,7 +22,8 @@ KX_EINVAL, KX_ESHAPE, KX_ETYPE, KX_EABI, KX_ELDS = -1, -2, -3, -4, -5
 
 EXPORTS = (
     "kx_version", "kx_last_error", "kx_workspace_bytes", "kx_encode_table",
-    "kx_tile_table", "kx_spread", "kx_gather", "kx_conv", "kx_forward",
+    "kx_tile_table", "kx_slot_table_elems", "kx_slot_table", "kx_spread",
+    "kx_gather", "kx_conv", "kx_forward", "kx_forward_work_bytes", "kx_forward_ws",
     "kx_adjoint", "kx_reduce_workspace_bytes", "kx_dot",
     "kx_solver_workspace_bytes", "kx_vec", "kx_dot_dev", "kx_lsqr_xw",
     "kx_cgls_scalar", "kx_lsqr_scalar", "kx_batch_dev_bytes", "kx_batch_build",
@@ -129,7 +130,7 @@ class KxPlan(ctypes.Structure):
         ("gsplit", ctypes.c_int32),
         ("sside", ctypes.c_int32),
         ("gtiles", ctypes.c_int32),
-        ("pad0", ctypes.c_int32),
+        ("slots", ctypes.c_int32),
         ("wtyp", ctypes.c_double),
     ]
 
@@ -190,6 +191,8 @@ def _declare(L):
         "kx_workspace_bytes": ([PP], I64),
         "kx_encode_table": ([PP, P, I32, D, I32, P, P, P], ctypes.c_int),
         "kx_tile_table": ([PP, P, I32, I32, P, P], ctypes.c_int),
+        "kx_slot_table_elems": ([PP, I32], I64),
+        "kx_slot_table": ([PP, I32, I32, P, P], ctypes.c_int),
         "kx_spread": ([PP, P, P, P], ctypes.c_int),
         "kx_gather": ([PP, P, P, P], ctypes.c_int),
         "kx_spread_models": ([PP, P, P, I32, P], ctypes.c_int),
@@ -198,6 +201,8 @@ def _declare(L):
         "kx_conv_rows": ([P, I64, P, I64, I32, P, I64, I32, I32, P], ctypes.c_int),
         "kx_xcorr_rows": ([P, I64, I32, P, I64, I32, P, I64, I32, I32, I32, P], ctypes.c_int),
         "kx_forward": ([PP, P, P, P, P], ctypes.c_int),
+        "kx_forward_work_bytes": ([PP], I64),
+        "kx_forward_ws": ([PP, P, P, P, I64, P], ctypes.c_int),
         "kx_adjoint": ([PP, P, P, P, P], ctypes.c_int),
         "kx_forward_noalloc": ([PP, P, P, P], ctypes.c_int),
         "kx_reduce_workspace_bytes": ([], I64),

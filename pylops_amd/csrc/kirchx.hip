@@ -192,6 +192,27 @@ __global__ __launch_bounds__(kBlock) void tile_kernel(KArgs a, const double *__r
         out[((size_t)t * n + j) * kWave + lane] = (TD)v;
 }
 
+// One 16-byte chunk of the slot-ordered copy per thread; receivers past the
+// last repeat it.
+template <typename TT>
+__global__ __launch_bounds__(kBlock) void slot_kernel(const TT *__restrict__ tab, int n,
+                                                      int64_t nchunk, TT *__restrict__ out)
+{
+    constexpr int CH = SlotChunkLen<TT>::v;
+    constexpr int per = kSlotBlock * kWave / CH;  // chunks of a (tile, block)
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= nchunk)
+        return;
+    const int64_t tb = i / per;
+    const int w = (int)(i % per);
+    const int nb = slot_blocks(n);
+    const int64_t t = tb / nb;
+    const int j = min((int)(tb % nb) * kSlotBlock + (w & 15), n - 1);
+    const int p = ((w >> 4) & 3) * 16 + (w >> 6) * CH;
+    reinterpret_cast<VecN<TT, CH> *>(out)[i] =
+        *reinterpret_cast<const VecN<TT, CH> *>(tab + (t * n + j) * kWave + p);
+}
+
 // ---------------------------------------------------------------------------
 // reductions (float64 accumulation)
 // ---------------------------------------------------------------------------
@@ -361,6 +382,40 @@ extern "C" int kx_tile_table(const kx_plan *geom, const double *tabT, int32_t n,
     return KX_OK;
 }
 
+extern "C" int64_t kx_slot_table_elems(const kx_plan *geom, int32_t n)
+{
+    if (check_geom(geom) || n <= 0)
+        return -1;
+    return (int64_t)slot_blocks(n) * kSlotBlock * geom->ntiles * kWave;
+}
+
+extern "C" int kx_slot_table(const kx_plan *geom, int32_t n, int32_t fmt, void *tab, void *stream)
+{
+    int rc = check_geom(geom);
+    if (rc)
+        return rc;
+    if (!tab || n <= 0)
+        return kx_fail(KX_EINVAL, "slot_table: bad arguments");
+    if (fmt != KX_F32 && fmt != KX_F16)
+        return kx_fail(KX_ETYPE, "slot_table: format %d", fmt);
+    const int64_t plain = (int64_t)n * geom->ntiles * kWave;
+    const int64_t nchunk = kx_slot_table_elems(geom, n) * (fmt == KX_F32 ? 4 : 2) / 16;
+    const int64_t nblk = (nchunk + kBlock - 1) / kBlock;
+    if (nblk > INT32_MAX)
+        return kx_fail(KX_ESHAPE, "slot_table: table too large");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (fmt == KX_F32)
+        hipLaunchKernelGGL(slot_kernel<float>, dim3((unsigned)nblk), dim3(kBlock), 0, st,
+                           reinterpret_cast<const float *>(tab), n, nchunk,
+                           reinterpret_cast<float *>(tab) + plain);
+    else
+        hipLaunchKernelGGL(slot_kernel<__half>, dim3((unsigned)nblk), dim3(kBlock), 0, st,
+                           reinterpret_cast<const __half *>(tab), n, nchunk,
+                           reinterpret_cast<__half *>(tab) + plain);
+    KX_LAUNCHED("slot_table");
+    return KX_OK;
+}
+
 extern "C" int kx_conv_rows(const void *x, int64_t xstride, void *y, int64_t ntr, int32_t nt,
                             const void *h, int64_t hstride, int32_t nh, int32_t dtype,
                             void *stream)
@@ -428,7 +483,21 @@ extern "C" int kx_xcorr_rows(const void *a, int64_t astride, int32_t la, const v
     return KX_OK;
 }
 
+extern "C" int64_t kx_forward_work_bytes(const kx_plan *p)
+{
+    const int64_t b = kx_workspace_bytes(p);
+    if (b < 0 || p->dtype != KX_F32 || !p->h || p->nh <= 0)
+        return b;
+    return std::max(b, kx_spread_sums_bytes(p));
+}
+
 extern "C" int kx_forward(const kx_plan *p, const void *m, void *d, void *work, void *stream)
+{
+    return kx_forward_ws(p, m, d, work, kx_workspace_bytes(p), stream);
+}
+
+extern "C" int kx_forward_ws(const kx_plan *p, const void *m, void *d, void *work,
+                             int64_t work_bytes, void *stream)
 {
     int rc = check_plan(p);
     if (rc)
@@ -437,8 +506,11 @@ extern "C" int kx_forward(const kx_plan *p, const void *m, void *d, void *work, 
         return kx_fail(KX_EINVAL, "forward: wavelet missing");
     if (!work)
         return kx_fail(KX_EINVAL, "forward: workspace missing");
+    if (work_bytes < kx_workspace_bytes(p))
+        return kx_fail(KX_EINVAL, "forward: workspace of %lld bytes, %lld needed",
+                       (long long)work_bytes, (long long)kx_workspace_bytes(p));
     // one launch where the workgroups can convolve their traces in LDS
-    rc = kx_spread_wavelet(p, m, d, stream);
+    rc = kx_spread_wavelet(p, m, d, work, work_bytes, stream);
     if (rc != KX_ENOFUSE)
         return rc;
     rc = kx_spread(p, m, work, stream);

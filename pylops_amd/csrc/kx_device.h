@@ -204,6 +204,23 @@ __device__ __forceinline__ int64_t point_index(const KArgs &a, const TilePoint &
 }
 
 // ---------------------------------------------------------------------------
+// slot-ordered receiver tables
+// ---------------------------------------------------------------------------
+// The copy behind a receiver table (kx_plan.slots): per tile and block of
+// kSlotBlock receivers, 16-byte chunks of consecutive points of one receiver,
+// chunk c of row group q (points 16 q + SlotChunkLen c ...) of receiver j at
+// chunk index (c 4 + q) 16 + j: lane 16 q + j of a wave reads chunk c of its
+// receiver next to its neighbours' (1 KB per load instruction).
+constexpr int kSlotBlock = 16;
+template <typename TT> struct SlotChunkLen {
+    static constexpr int v = 16 / (int)sizeof(TT);
+};
+__host__ __device__ __forceinline__ int slot_blocks(int n)
+{
+    return (n + kSlotBlock - 1) / kSlotBlock;
+}
+
+// ---------------------------------------------------------------------------
 // forward: spread into LDS-resident traces
 // ---------------------------------------------------------------------------
 // LDS accumulation.  For float data every contribution c (rounded to float
@@ -467,14 +484,16 @@ __device__ __forceinline__ void spread_sample(TC T, int base, TD w, bool on, int
         }
         const TD w1 = w * (TD)f;
         if constexpr (ACC == kAccFix) {
-            // w (1 - f) in one rounding; fixed point by floor(x + 1/2) in
-            // one conversion
+            // fixed point by floor(x + 1/2) in one conversion; the first
+            // sample takes what the second leaves of the rounded weight, so
+            // that the pair's sum is the weight's own rounding
             unsigned long long *acci = static_cast<unsigned long long *>(lds);
-            const TD w0 = fma(-w, (TD)f, w);
+            const int i1 = round_half_up(w1);
+            const int i0 = round_half_up(w) - i1;
             if (in0)
-                atomicAdd(&acci[it], (unsigned long long)(long long)round_half_up(w0));
+                atomicAdd(&acci[it], (unsigned long long)(long long)i0);
             if (in1)
-                atomicAdd(&acci[it + 1], (unsigned long long)(long long)round_half_up(w1));
+                atomicAdd(&acci[it + 1], (unsigned long long)(long long)i1);
         } else {
             double *accd = static_cast<double *>(lds);
             const TD w0 = w * (TD)(TC(1) - f);
@@ -614,6 +633,52 @@ inline bool fused_conv_ok(int rb, int nt, int nh, size_t lds, int block)
     return true;
 }
 
+// Convolves the nrl float rows at win (x[p - L] at position p of row j, S =
+// fused_row(nt, nh) floats apart, written by the workgroup before the call)
+// and writes row j to trace first + j * trb of y: kx_conv's operations in
+// kx_conv's order.
+__device__ __forceinline__ void rows_conv_store(float *__restrict__ win, float *__restrict__ y,
+                                                size_t first, int trb, int nt, int nrl,
+                                                const float *__restrict__ h, int nh)
+{
+    const int S = fused_row(nt, nh), L = (nh - 1) / 2, nhp = conv_taps_padded(nh);
+    // zero margins of the rows, then the flipped filter
+    const int F = nrl * S;
+    for (int p = threadIdx.x; p < F; p += blockDim.x) {
+        const int n = p % S - L;
+        if (n < 0 || n >= nt)
+            win[p] = 0.f;
+    }
+    for (int k = threadIdx.x; k < nhp; k += blockDim.x)
+        win[F + k] = k < nh ? h[nh - 1 - k] : 0.f;
+    __syncthreads();
+    const int G = (nt + 3) / 4;  // groups of 4 outputs per row
+    const float4 *h4 = reinterpret_cast<const float4 *>(win + F);
+    for (int g = threadIdx.x; g < nrl * G; g += blockDim.x) {
+        const int j = g / G, n0 = (g - j * G) * 4;
+        const float4 *w4 = reinterpret_cast<const float4 *>(win + j * S + n0);
+        float acc[kConvPer] = {};
+        float4 cur = w4[0];
+        for (int gq = 0; gq < nhp / 4; ++gq) {
+            const float4 nxt = w4[gq + 1];
+            const float4 hq = h4[gq];
+            const float w[8] = {cur.x, cur.y, cur.z, cur.w, nxt.x, nxt.y, nxt.z, nxt.w};
+            const float hh[4] = {hq.x, hq.y, hq.z, hq.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int r = 0; r < kConvPer; ++r)
+                    acc[r] += hh[q] * w[q + r];
+            cur = nxt;
+        }
+        float *yo = y + (first + (size_t)j * trb) * nt;
+#pragma unroll
+        for (int r = 0; r < kConvPer; ++r)
+            if (n0 + r < nt)
+                yo[n0 + r] = acc[r];
+    }
+}
+
 template <typename TD, int ACC>
 __device__ __forceinline__ void traces_conv_store(TD *__restrict__ y, size_t first, int trb,
                                                   int nt, int nrl, int e, void *lds,
@@ -621,7 +686,7 @@ __device__ __forceinline__ void traces_conv_store(TD *__restrict__ y, size_t fir
 {
     if constexpr (sizeof(TD) == 4) {
         const int ntr = nrl * nt, lts = trace_stride(nt);
-        const int S = fused_row(nt, nh), L = (nh - 1) / 2, nhp = conv_taps_padded(nh);
+        const int S = fused_row(nt, nh), L = (nh - 1) / 2;
         float *win = static_cast<float *>(lds);
         const unsigned long long *acci = static_cast<const unsigned long long *>(lds);
         const double *accd = static_cast<const double *>(lds);
@@ -650,41 +715,7 @@ __device__ __forceinline__ void traces_conv_store(TD *__restrict__ y, size_t fir
             }
             __syncthreads();
         }
-        // zero margins of the rows, then the flipped filter
-        const int F = nrl * S;
-        for (int p = threadIdx.x; p < F; p += blockDim.x) {
-            const int n = p % S - L;
-            if (n < 0 || n >= nt)
-                win[p] = 0.f;
-        }
-        for (int k = threadIdx.x; k < nhp; k += blockDim.x)
-            win[F + k] = k < nh ? h[nh - 1 - k] : 0.f;
-        __syncthreads();
-        const int G = (nt + 3) / 4;  // groups of 4 outputs per row
-        const float4 *h4 = reinterpret_cast<const float4 *>(win + F);
-        for (int g = threadIdx.x; g < nrl * G; g += blockDim.x) {
-            const int j = g / G, n0 = (g - j * G) * 4;
-            const float4 *w4 = reinterpret_cast<const float4 *>(win + j * S + n0);
-            float acc[kConvPer] = {};
-            float4 cur = w4[0];
-            for (int gq = 0; gq < nhp / 4; ++gq) {
-                const float4 nxt = w4[gq + 1];
-                const float4 hq = h4[gq];
-                const float w[8] = {cur.x, cur.y, cur.z, cur.w, nxt.x, nxt.y, nxt.z, nxt.w};
-                const float hh[4] = {hq.x, hq.y, hq.z, hq.w};
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-#pragma unroll
-                    for (int r = 0; r < kConvPer; ++r)
-                        acc[r] += hh[q] * w[q + r];
-                cur = nxt;
-            }
-            TD *yo = y + (first + (size_t)j * trb) * nt;
-#pragma unroll
-            for (int r = 0; r < kConvPer; ++r)
-                if (n0 + r < nt)
-                    yo[n0 + r] = acc[r];
-        }
+        rows_conv_store(win, y, first, trb, nt, nrl, h, nh);
         __syncthreads();  // the rows are read before a next item clears them
     } else {
         traces_store<TD, ACC>(y, first, trb, nt, trace_stride(nt), nrl, e, lds);
@@ -904,9 +935,10 @@ __device__ __forceinline__ void models_accumulate(const ModelsTile<TT, K> &cur, 
             const int it = j * nt + k;
             const float w1 = w * f;
             if constexpr (FIX) {
-                const float w0 = fmaf(-w, f, w);
-                atomicAdd(&acci[it], (unsigned long long)(long long)round_half_up(w0));
-                atomicAdd(&acci[it + 1], (unsigned long long)(long long)round_half_up(w1));
+                const int i1 = round_half_up(w1);
+                const int i0 = round_half_up(w) - i1;
+                atomicAdd(&acci[it], (unsigned long long)(long long)i0);
+                atomicAdd(&acci[it + 1], (unsigned long long)(long long)i1);
             } else {
                 const float w0 = w * (1.f - f);
                 atomicAdd(&accd[it], (double)w0);
@@ -1019,15 +1051,15 @@ __device__ __forceinline__ void stats_block(const float *__restrict__ m, int64_t
     }
 }
 
-// The np partial statistics combined by one wave (sums in float64): the
-// maximum and the mean of the nonzero |m| (0 without any); valid in every
-// lane.
+// The np partial statistics combined by every wave of the workgroup for
+// itself (sums in float64): the maximum and the mean of the nonzero |m| (0
+// without any); valid in every lane.
 __device__ __forceinline__ void stats_wave(const float *__restrict__ part, int np, float &mx,
                                            double &mean)
 {
     float x = 0.f;
     double sum = 0.0, cnt = 0.0;
-    for (int i = threadIdx.x; i < np; i += kWave) {
+    for (int i = threadIdx.x & (kWave - 1); i < np; i += kWave) {
         x = fmaxf(x, part[i]);
         sum += part[np + i];
         cnt += part[2 * np + i];

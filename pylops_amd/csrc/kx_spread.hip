@@ -5,11 +5,13 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <mutex>
 
 #include "kx_internal.h"
 #include "kx_device.h"
+#include "kx_slots.h"
 
 namespace {
 
@@ -24,6 +26,93 @@ __global__ __launch_bounds__(kSpreadBlock) void spread_kernel(KArgs a, const TD 
     const int L = xcd_remap(blockIdx.x, gridDim.x);
     const SpreadScale scale = *sc;
     spread_item<TD, TT, DYN, NEG, ORD, RB, XS>(a, m, y, scale, L % a.ns, (L / a.ns) * RB, h, nh);
+}
+
+// Blocks of 8 or 16 receivers, interleaved traces (kx_slots.h).  The first
+// nfull workgroups take a whole (source, receiver block) pair each, pair L
+// (after the XCD renumbering) = source L mod ns, block L / ns; each of the
+// remaining pairs is shared by `parts` workgroups, pair nfull + (L mod nrest),
+// part L / nrest of the tiles: neighbours read the same rows of the receiver
+// tables.  Every wave turns the np partial statistics of |m| into the
+// launch's scale for itself (one launch less than a kernel for it);
+// workgroup 0 keeps it in *sc.
+struct SlotsLaunch {
+    const float *part;
+    int np;
+    double wamp, wtyp;
+    SpreadScale *sc;
+    int nfull, parts;
+    unsigned long long *sums;  // [parts][nrest][nt][RB]
+};
+
+template <typename TT, bool DYN, bool GATE, bool NEG, int RB>
+__global__ __launch_bounds__(kSlotsMaxThreads) void slots_kernel(KArgs a,
+                                                                 const float *__restrict__ m,
+                                                                 float *__restrict__ y,
+                                                                 const float *__restrict__ h,
+                                                                 int nh, SlotsLaunch g)
+{
+    float mx;
+    double mean;
+    stats_wave(g.part, g.np, mx, mean);
+    SpreadScale scale = scale_from_stats(mx, mean, g.wamp, g.wtyp);
+    scale.e = __builtin_amdgcn_readfirstlane(scale.e);
+    scale.fixed = __builtin_amdgcn_readfirstlane(scale.fixed);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *g.sc = scale;
+    int pair, t0 = 0, t1 = a.ntiles;
+    SlotsOut out{y, h, nh, nullptr};
+    if ((int)blockIdx.x < g.nfull) {
+        pair = xcd_remap(blockIdx.x, g.nfull);
+    } else {
+        const int nrest = (int)(gridDim.x - g.nfull) / g.parts;
+        const int L = xcd_remap(blockIdx.x - g.nfull, gridDim.x - g.nfull);
+        const int part = L / nrest;
+        pair = g.nfull + L % nrest;
+        t0 = (int)((int64_t)a.ntiles * part / g.parts);
+        t1 = (int)((int64_t)a.ntiles * (part + 1) / g.parts);
+        if (g.parts > 1)
+            out.sums = g.sums + (size_t)L * a.nt * RB;
+    }
+    slots_item<TT, DYN, GATE, NEG, RB>(a, m, scale, pair % a.ns, (pair / a.ns) * RB, t0, t1, out);
+}
+
+// The parts of a pair added, converted and convolved: workgroup b = four
+// slots (b mod (rb / 4)) of pair nfull + b / (rb / 4).
+constexpr int kFinalRows = 4;
+__global__ __launch_bounds__(kBlock) void slots_final_kernel(KArgs a, int rb, SlotsLaunch g,
+                                                             int nrest, float *__restrict__ y,
+                                                             const float *__restrict__ h, int nh)
+{
+    extern __shared__ __align__(16) unsigned char kx_smem[];
+    float *win = reinterpret_cast<float *>(kx_smem);
+    const SpreadScale scale = *g.sc;
+    const int nq = rb / kFinalRows;
+    const int j0 = (int)(blockIdx.x % nq) * kFinalRows, rest = (int)blockIdx.x / nq;
+    const int pair = g.nfull + rest;
+    const int s = pair % a.ns, r0 = (pair / a.ns) * rb + j0;
+    const int nrl = min(kFinalRows, a.nr - r0);
+    if (nrl <= 0)
+        return;  // uniform over the workgroup
+    const int S = fused_row(a.nt, nh), Lm = (nh - 1) / 2;
+    const size_t block = (size_t)a.nt * rb, stride = (size_t)nrest * block;
+    const unsigned long long *p = g.sums + rest * block + j0;
+    for (int i = threadIdx.x; i < a.nt * kFinalRows; i += kBlock) {
+        const int j = i & (kFinalRows - 1), n = i / kFinalRows;
+        const unsigned long long *q = p + (size_t)n * rb + j;
+        unsigned long long acc = 0;
+        double accd = 0.0;
+#pragma unroll 4
+        for (int k = 0; k < g.parts; ++k) {
+            const unsigned long long v = q[k * stride];
+            acc += v;
+            accd += __builtin_bit_cast(double, v);
+        }
+        if (j < nrl)
+            win[j * S + Lm + n] =
+                scale.fixed ? (float)ldexp((double)(long long)acc, -scale.e) : (float)accd;
+    }
+    rows_conv_store(win, y, (size_t)s * a.nr + r0, 1, a.nt, nrl, h, nh);
 }
 
 // Traces longer than a workgroup's LDS: workgroup L (after the XCD
@@ -65,7 +154,19 @@ __global__ __launch_bounds__(kSpreadBlock) void spread_models_kernel(
         spread_models_body<TT, DYN, NEG, false, K>(a, m, ni, y, ystride, sc, L % a.ns, L / a.ns);
 }
 
-constexpr int kRblocks[] = {16, 8, 4, 2, 1};
+constexpr int kRblocks[] = {4, 2, 1};
+
+int device_cus()
+{
+    int cus = 256, dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        (void)hipGetLastError();
+        cus = 256;
+    }
+    return cus;
+}
+
 constexpr int kLdsPerCu = 160 * 1024;
 constexpr int kMaxWavesPerCu = 32;
 
@@ -96,10 +197,6 @@ template <typename TD, typename TT, bool DYN, bool NEG, bool XS, int ORD>
 const void *spread_fn(int rb)
 {
     switch (rb) {
-    case 16:
-        return reinterpret_cast<const void *>(&spread_kernel<TD, TT, DYN, NEG, ORD, 16, XS>);
-    case 8:
-        return reinterpret_cast<const void *>(&spread_kernel<TD, TT, DYN, NEG, ORD, 8, XS>);
     case 4:
         return reinterpret_cast<const void *>(&spread_kernel<TD, TT, DYN, NEG, ORD, 4, XS>);
     case 2:
@@ -165,10 +262,6 @@ int launch_spread_o(KArgs a, int requested, int max_rb, const void *m, void *y,
 {
     a.rblock = pick_rblock<TD, TT, DYN, NEG, XS, ORD>(requested, a.nr, a.nt, max_rb);
     switch (a.rblock) {
-    case 16:
-        return launch_spread_rb<TD, TT, DYN, NEG, XS, ORD, 16>(a, m, y, sc, st, h, nh);
-    case 8:
-        return launch_spread_rb<TD, TT, DYN, NEG, XS, ORD, 8>(a, m, y, sc, st, h, nh);
     case 4:
         return launch_spread_rb<TD, TT, DYN, NEG, XS, ORD, 4>(a, m, y, sc, st, h, nh);
     case 2:
@@ -176,6 +269,113 @@ int launch_spread_o(KArgs a, int requested, int max_rb, const void *m, void *y,
     default:
         return launch_spread_rb<TD, TT, DYN, NEG, XS, kOrdNatural, 1>(a, m, y, sc, st, h, nh);
     }
+}
+
+// How a forward runs in slot blocks: rb receivers per workgroup (0: the
+// kernels of 4, 2 and 1), the pairs past the first nfull in `parts`
+// workgroups each.
+struct SlotsShape {
+    int rb, threads, nfull, parts;
+    size_t lds, sums_bytes;
+};
+
+// The shape with the smallest estimated time, in clocks of a CU.  A CU's
+// clocks per tile and receiver, with all its waves, were measured at: blocks
+// of 4, 2 or 1 27 kinematic and 36 dynamic; slots of 16 17 (float32 tables,
+// 3D 128x128x120 with 25 x 400) and 15 (float16), dynamic 30 (2D 201x121
+// with 21 x 101; float16 333x187 with 37 x 149); slots of 8 a quarter more,
+// dynamic 32 (601x300 with 61 x 301).  A workgroup spends about 18000
+// clocks on its scale, first loads, clearing and writing out.  Where the
+// pairs are no multiple of the workgroups that run at once, the last ones are
+// shared by several workgroups, which costs their sums' way through memory
+// (about 1000 bytes per clock).  The estimates miss by up to 8%: the slots have
+// to gain as much.  A requested block size is an upper bound.
+SlotsShape pick_slots(const kx_plan *p, int nh, int64_t work_bytes)
+{
+    SlotsShape best{0, 0, 0, 1, 0, 0};
+    if (!p->slots || p->dtype != KX_F32 || p->sside == KX_SIDE_SOURCES)
+        return best;
+    const int cus = device_cus();
+    const bool half = p->tab_fmt == KX_F16;
+    const double fixed = 18000.0, tiles = (double)p->ntiles;
+    double best_t = 1e300;
+    if (p->rblock == 0) {  // what the kernels of 4 would take
+        const double pairs = (double)p->ns * ((p->nr + 3) / 4);
+        best_t = 0.92 * (std::ceil(pairs / cus) * tiles * 4 * (p->dynamic ? 36.0 : 27.0) + fixed);
+    }
+    for (int rb : {16, 8}) {
+        if (p->rblock > 0 && rb > p->rblock)
+            continue;
+        const int th = slots_threads(rb, p->nt, nh);
+        if (!th)
+            continue;
+        const int per_cu = kSlotsMaxThreads / th, at_once = cus * per_cu;
+        const int64_t pairs = (int64_t)p->ns * ((p->nr + rb - 1) / rb);
+        const double step = p->dynamic ? (rb == 8 ? 32.0 : 30.0)
+                                       : (half ? 15.0 : 17.0) * (rb == 8 ? 1.25 : 1.0);
+        const double work = tiles * rb * step * per_cu, c0 = fixed + p->nt * rb / th * 60.0;
+        for (int parts = 1; parts <= 16; ++parts) {
+            const int64_t nfull = parts > 1 ? pairs / at_once * at_once : pairs;
+            const int64_t nrest = pairs - nfull;
+            const size_t sums = parts > 1 ? (size_t)(nrest * parts) * p->nt * rb * 8 : 0;
+            if (parts > 1 && (nh <= 0 || nrest == 0 || (int64_t)sums > work_bytes ||
+                              p->ntiles < (int64_t)parts * (th / kWave)))
+                break;
+            double t = std::ceil((double)nfull / at_once) * (work + c0);
+            if (parts > 1)
+                t += std::ceil((double)nrest * parts / at_once) * (work / parts + c0) + 15000.0 +
+                     2.0 * sums / 1000.0;
+            if (t < best_t * 0.98) {
+                best_t = t;
+                best = {rb, th, (int)nfull, parts, slots_lds_bytes(rb, p->nt, nh), sums};
+            }
+        }
+    }
+    return best;
+}
+
+template <typename TT, bool DYN, bool GATE, bool NEG, int RB>
+int launch_slots_rb(const KArgs &a, const SlotsShape &g, const SlotsLaunch &l, const void *m,
+                    void *y, hipStream_t st, const void *h, int nh)
+{
+    const int nrest = a.ns * ((a.nr + RB - 1) / RB) - g.nfull;
+    allow_lds(reinterpret_cast<const void *>(&slots_kernel<TT, DYN, GATE, NEG, RB>), g.lds);
+    hipLaunchKernelGGL((slots_kernel<TT, DYN, GATE, NEG, RB>), dim3(g.nfull + nrest * g.parts),
+                       dim3(g.threads), g.lds, st, a, reinterpret_cast<const float *>(m),
+                       reinterpret_cast<float *>(y), reinterpret_cast<const float *>(h), nh, l);
+    KX_LAUNCHED("spread");
+    if (g.parts > 1) {
+        const size_t lds =
+            ((size_t)kFinalRows * fused_row(a.nt, nh) + conv_taps_padded(nh)) * sizeof(float);
+        allow_lds(reinterpret_cast<const void *>(&slots_final_kernel), lds);
+        hipLaunchKernelGGL(slots_final_kernel, dim3(nrest * (RB / kFinalRows)), dim3(kBlock), lds,
+                           st, a, RB, l, nrest, reinterpret_cast<float *>(y),
+                           reinterpret_cast<const float *>(h), nh);
+        KX_LAUNCHED("spread parts");
+    }
+    return KX_OK;
+}
+
+template <typename TT, bool DYN, bool GATE, bool NEG>
+int launch_slots(const KArgs &a, const SlotsShape &g, const SlotsLaunch &l, const void *m,
+                 void *y, hipStream_t st, const void *h, int nh)
+{
+    return g.rb == 16 ? launch_slots_rb<TT, DYN, GATE, NEG, 16>(a, g, l, m, y, st, h, nh)
+                      : launch_slots_rb<TT, DYN, GATE, NEG, 8>(a, g, l, m, y, st, h, nh);
+}
+
+template <typename TT>
+int launch_slots_d(const kx_plan *p, const KArgs &a, const SlotsShape &g, const SlotsLaunch &l,
+                   const void *m, void *y, hipStream_t st, const void *h, int nh)
+{
+    if (p->dynamic == KX_DYNAMIC_NOGATE)
+        return p->neg_trav ? launch_slots<TT, true, false, true>(a, g, l, m, y, st, h, nh)
+                           : launch_slots<TT, true, false, false>(a, g, l, m, y, st, h, nh);
+    if (p->dynamic)
+        return p->neg_trav ? launch_slots<TT, true, true, true>(a, g, l, m, y, st, h, nh)
+                           : launch_slots<TT, true, true, false>(a, g, l, m, y, st, h, nh);
+    return p->neg_trav ? launch_slots<TT, false, false, true>(a, g, l, m, y, st, h, nh)
+                       : launch_slots<TT, false, false, false>(a, g, l, m, y, st, h, nh);
 }
 
 template <typename TD, typename TT, bool DYN, bool NEG, bool XS>
@@ -226,9 +426,10 @@ int launch_spread_seg(const KArgs &a, const void *m, void *y, const SpreadScale 
     return KX_OK;
 }
 
+// work: work_bytes of scratch for the parts of slot blocks (0: one part).
 template <typename TD, typename TT>
 int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream_t st,
-                    const void *h = nullptr)
+                    const void *h = nullptr, void *work = nullptr, int64_t work_bytes = 0)
 {
     const int nh = h != nullptr ? p->nh : 0;
     if (h != nullptr && sizeof(TD) != 4)
@@ -241,15 +442,16 @@ int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream
     if (sizeof(TD) == 4 && !p->aux)
         return kx_failf(KX_EINVAL, "spread: plan.aux (KX_AUX_BYTES of device scratch) is NULL");
     // registers per lane grow with the block: keep two workgroups per CU
-    const int max_rb = sizeof(TD) == 8 ? 4 : (p->dynamic ? 8 : 16);
+    const int max_rb = 4;
     SpreadScale *sc = reinterpret_cast<SpreadScale *>(p->aux);
+    const SlotsShape slots = pick_slots(p, nh, work ? work_bytes : 0);
     int side = p->sside;
     if (side == KX_SIDE_AUTO)
         side = (p->ny == 1 && p->ns < p->nr) ? KX_SIDE_SOURCES : KX_SIDE_RECEIVERS;
     // (float16 plans keep the two sides' offsets in different types and
     // block receivers)
     const bool xs = sizeof(TD) == 4 && side == KX_SIDE_SOURCES && p->tab_fmt != KX_F16;
-    if (sizeof(TD) == 4) {
+    if constexpr (sizeof(TD) == 4) {
         // fixed-point scale of this launch from max|m|
         const int64_t ni = (int64_t)p->nx * p->ny * p->nz;
         float *part = reinterpret_cast<float *>(p->aux) + 16;
@@ -257,6 +459,11 @@ int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream
         hipLaunchKernelGGL(absmax_partial_kernel, dim3(nb), dim3(kBlock), 0, st,
                            reinterpret_cast<const float *>(m), ni, part);
         KX_LAUNCHED("spread scale");
+        if (slots.rb) {
+            const SlotsLaunch l{part, nb, p->wamp, p->wtyp, sc, slots.nfull, slots.parts,
+                                static_cast<unsigned long long *>(work)};
+            return launch_slots_d<TT>(p, a, slots, l, m, y, st, h, nh);
+        }
         hipLaunchKernelGGL(scale_final_kernel, dim3(1), dim3(kWave), 0, st, part, nb, p->wamp,
                            p->wtyp, sc);
         KX_LAUNCHED("spread scale");
@@ -323,9 +530,8 @@ extern "C" int kx_spread(const kx_plan *p, const void *m, void *traces, void *st
     return launch_spread_d<float, float>(p, a, m, traces, st);
 }
 
-extern "C" __attribute__((visibility("hidden"))) int kx_spread_wavelet(const kx_plan *p,
-                                                                      const void *m, void *d,
-                                                                      void *stream)
+extern "C" __attribute__((visibility("hidden"))) int kx_spread_wavelet(
+    const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes, void *stream)
 {
     int rc = kx_plan_check(p);
     if (rc)
@@ -337,8 +543,13 @@ extern "C" __attribute__((visibility("hidden"))) int kx_spread_wavelet(const kx_
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const KArgs a = make_args(p);
     if (p->tab_fmt == KX_F16)
-        return launch_spread_d<float, __half>(p, a, m, d, st, p->h);
-    return launch_spread_d<float, float>(p, a, m, d, st, p->h);
+        return launch_spread_d<float, __half>(p, a, m, d, st, p->h, work, work_bytes);
+    return launch_spread_d<float, float>(p, a, m, d, st, p->h, work, work_bytes);
+}
+
+extern "C" __attribute__((visibility("hidden"))) int64_t kx_spread_sums_bytes(const kx_plan *p)
+{
+    return (int64_t)pick_slots(p, p->nh, INT64_MAX).sums_bytes;
 }
 
 namespace {
@@ -495,7 +706,7 @@ extern "C" int kx_forward_noalloc(const kx_plan *p, const void *m, void *d, void
     // clearing)
     kx_plan q = *p;
     q.aux = s;
-    rc = kx_spread_wavelet(&q, m, d, stream);
+    rc = kx_spread_wavelet(&q, m, d, nullptr, 0, stream);
     if (rc == KX_ENOFUSE)
         return kx_failf(KX_ELDS,
                         "forward_noalloc: this plan's forward cannot convolve in the spread "

@@ -256,7 +256,22 @@ def make_geom_plan(nx, ny, nz, tile):
     return p
 
 
-def encode(plan, tab, scale, fmt, lo=-math.inf, hi=math.inf):
+def _empty_table(plan, n, tdt, device, slots):
+    """(buffer, view of its (ntiles, n, 64) table): with ``slots`` the buffer
+    has room behind the table for its slot-ordered copy."""
+    elems = plan.ntiles * n * 64
+    extra = _lib.load().kx_slot_table_elems(ctypes.byref(plan), n) if slots else 0
+    buf = torch.empty(elems + extra, dtype=tdt, device=device)
+    return buf, buf[:elems].view(plan.ntiles, n, 64)
+
+
+def _fill_slots(plan, n, fmt, buf):
+    rc = _lib.load().kx_slot_table(ctypes.byref(plan), n, fmt, _lib.ptr(buf),
+                                   _lib.stream_ptr(buf.device))
+    _lib.check(rc, "kx_slot_table")
+
+
+def encode(plan, tab, scale, fmt, lo=-math.inf, hi=math.inf, slots=False):
     """tab: float64 device tensor (ni, n) in reference order -> (off, base)
     device tensors in the tiled layout, offsets in samples (tab*scale).
 
@@ -264,7 +279,10 @@ def encode(plan, tab, scale, fmt, lo=-math.inf, hi=math.inf):
     (the caller derives the bounds from the other side's extreme times);
     they are passed to the encoder as NaN, which gives them an offset far
     outside every trace and leaves them out of their tile's base, so that
-    unreachable points (huge times) cost the others no precision."""
+    unreachable points (huge times) cost the others no precision.
+
+    ``slots``: the offsets are followed in memory by their slot-ordered copy
+    (``kx_slot_table``, which the forward's receiver blocks read)."""
     n = tab.shape[1]
     if not bool(torch.isfinite(tab).all()):
         raise ValueError("traveltime table contains non-finite values")
@@ -275,23 +293,28 @@ def encode(plan, tab, scale, fmt, lo=-math.inf, hi=math.inf):
     tabT = tab.t().contiguous()
     tdt = {_lib.KX_F32: torch.float32, _lib.KX_F16: torch.float16,
            _lib.KX_F64: torch.float64}[fmt]
-    off = torch.empty((plan.ntiles, n, 64), dtype=tdt, device=tab.device)
+    buf, off = _empty_table(plan, n, tdt, tab.device, slots)
     base = torch.empty((plan.ntiles, n), dtype=torch.int32, device=tab.device)
     rc = _lib.load().kx_encode_table(ctypes.byref(plan), _lib.ptr(tabT), n, float(scale), fmt,
                                      _lib.ptr(off), _lib.ptr(base), _lib.stream_ptr(tab.device))
     _lib.check(rc, "kx_encode_table")
+    if slots:
+        _fill_slots(plan, n, fmt, buf)
     return off, base
 
 
-def tile(plan, tab, fmt):
-    """float64 (ni, n) -> [ntiles][n][64] of dtype fmt, zero padded."""
+def tile(plan, tab, fmt, slots=False):
+    """float64 (ni, n) -> [ntiles][n][64] of dtype fmt, zero padded;
+    ``slots`` as in :func:`encode`."""
     n = tab.shape[1]
     tabT = tab.t().contiguous()
     tdt = {_lib.KX_F64: torch.float64, _lib.KX_F16: torch.float16}.get(fmt, torch.float32)
-    out = torch.empty((plan.ntiles, n, 64), dtype=tdt, device=tab.device)
+    buf, out = _empty_table(plan, n, tdt, tab.device, slots)
     rc = _lib.load().kx_tile_table(ctypes.byref(plan), _lib.ptr(tabT), n, fmt, _lib.ptr(out),
                                    _lib.stream_ptr(tab.device))
     _lib.check(rc, "kx_tile_table")
+    if slots:
+        _fill_slots(plan, n, fmt, buf)
     return out
 
 

@@ -388,7 +388,10 @@ class Kirchhoff(LinearOperator):
         keep["off_s"], keep["base_s"] = T.encode(plan, ts, inv_dt,
                                                  _lib.KX_F32 if fmt == _lib.KX_F16 else fmt,
                                                  lo_s, hi_s)
-        keep["off_r"], keep["base_r"] = T.encode(plan, tr, inv_dt, fmt, lo_r, hi_r)
+        # float32 operators: the forward's receiver blocks read slot-ordered
+        # copies of the receiver tables
+        slots = self.dtype == np.float32
+        keep["off_r"], keep["base_r"] = T.encode(plan, tr, inv_dt, fmt, lo_r, hi_r, slots)
         del ts, tr
         wfmt = _lib.KX_F64 if self.dtype == np.float64 else _lib.KX_F32
         if self.dynamic:
@@ -411,8 +414,8 @@ class Kirchhoff(LinearOperator):
                 rfmt = _lib.KX_F16
             keep["wp_s"] = T.tile(plan, ps, wfmt)
             keep["wq_s"] = T.tile(plan, qs, wfmt)
-            keep["wp_r"] = T.tile(plan, pr, rfmt)
-            keep["wq_r"] = T.tile(plan, qr, rfmt)
+            keep["wp_r"] = T.tile(plan, pr, rfmt, slots)
+            keep["wq_r"] = T.tile(plan, qr, rfmt, slots)
             # |ps pr + qs qr| <= |(ps, qs)| |(pr, qr)|: bounds every weight
             plan.wamp = T.weight_bound(keep["wp_s"], keep["wq_s"]) * \
                 T.weight_bound(keep["wp_r"], keep["wq_r"])
@@ -445,6 +448,7 @@ class Kirchhoff(LinearOperator):
             plan.dynamic = _lib.KX_DYNAMIC_NOGATE
         plan.ns, plan.nr, plan.nt = ns, nr, self.nt
         plan.neg_trav = int(neg)
+        plan.slots = int(slots)
         plan.rblock = self.rblock
         plan.sorder = self.sorder
         plan.sside = self.sside
@@ -455,6 +459,7 @@ class Kirchhoff(LinearOperator):
             setattr(plan, k, v.data_ptr())
         object.__setattr__(self, "_dev_tables", keep)
         object.__setattr__(self, "_plan", plan)
+        object.__setattr__(self, "_ws_key", None)
         object.__setattr__(self, "_dirty", False)
 
     @property
@@ -464,8 +469,27 @@ class Kirchhoff(LinearOperator):
             self._build_device_tables()
         return self._plan
 
-    def _work(self, device, tdtype):
-        return torch.empty(self.nsnr * self.nt, dtype=tdtype, device=device)
+    def _work_bytes(self, plan):
+        """Workspace with which the products run fastest, found again when a
+        launch attribute changed."""
+        key = (plan.rblock, plan.sside)
+        if getattr(self, "_ws_key", None) != key:
+            n = max(int(_lib.load().kx_forward_work_bytes(ctypes.byref(plan))),
+                    self.nsnr * self.nt * self.dtype.itemsize)
+            object.__setattr__(self, "_ws_bytes", n)
+            object.__setattr__(self, "_ws_key", key)
+        return self._ws_bytes
+
+    def _product(self, plan, x, out, work, adjoint):
+        """Enqueue out <- Op x (Op^H x) on contiguous device tensors."""
+        L = _lib.load()
+        st = _lib.stream_ptr(x.device)
+        if adjoint:
+            _lib.check(L.kx_adjoint(ctypes.byref(plan), _lib.ptr(x), _lib.ptr(out),
+                                    _lib.ptr(work), st), "kx_adjoint")
+        else:
+            _lib.check(L.kx_forward_ws(ctypes.byref(plan), _lib.ptr(x), _lib.ptr(out),
+                                       _lib.ptr(work), work.numel(), st), "kx_forward_ws")
 
     def _into(self, x, out, adjoint):
         """Device fast path for the solvers: apply the operator (adjoint if
@@ -474,28 +498,23 @@ class Kirchhoff(LinearOperator):
         iteration always touches the same buffers."""
         plan = self.plan
         ws = getattr(self, "_ws", None)
-        if ws is None or ws.dtype != x.dtype or ws.device != x.device:
-            ws = torch.empty(self.nsnr * self.nt, dtype=x.dtype, device=x.device)
+        nws = self._work_bytes(plan)
+        if ws is None or ws.numel() < nws or ws.device != x.device:
+            ws = torch.empty(nws, dtype=torch.uint8, device=x.device)
             object.__setattr__(self, "_ws", ws)
-        L = _lib.load()
-        fn = L.kx_adjoint if adjoint else L.kx_forward
-        rc = fn(ctypes.byref(plan), _lib.ptr(x), _lib.ptr(out), _lib.ptr(ws),
-                _lib.stream_ptr(x.device))
-        _lib.check(rc, "kx_adjoint" if adjoint else "kx_forward")
+        self._product(plan, x, out, ws, adjoint)
         if adjoint:
             self.rmatvec_count += 1
         else:
             self.matvec_count += 1
         return out
 
-    def _launch(self, fn, x, nout, what):
+    def _launch(self, x, nout, adjoint):
         plan = self.plan
         xd = to_device(x.reshape(-1), self.dtype, self.device)
         out = torch.empty(nout, dtype=xd.dtype, device=self.device)
-        work = self._work(self.device, xd.dtype)
-        rc = fn(ctypes.byref(plan), _lib.ptr(xd), _lib.ptr(out), _lib.ptr(work),
-                _lib.stream_ptr(self.device))
-        _lib.check(rc, what)
+        work = torch.empty(self._work_bytes(plan), dtype=torch.uint8, device=self.device)
+        self._product(plan, xd, out, work, adjoint)
         return like_input(out, x)
 
     # ------------------------------------------------------------------
@@ -516,7 +535,7 @@ class Kirchhoff(LinearOperator):
             # (the reference's scipy upcast, C1D:99-106): float64 data
             traces = self.spread(to_device(x.reshape(-1), self.dtype, self.device))
             return like_input(self._conv64(traces.double(), self._dev_tables["h64"]), x)
-        return self._launch(_lib.load().kx_forward, x, self.nsnr * self.nt, "kx_forward")
+        return self._launch(x, self.nsnr * self.nt, False)
 
     @reshaped
     def _rmatvec(self, x):
@@ -526,7 +545,7 @@ class Kirchhoff(LinearOperator):
             xd = to_device(x.reshape(-1), np.float64, self.device)
             dc = self._conv64(xd, self._dev_tables["hstar64"])
             return like_input(self.gather(dc.to(torch.float32)), x)
-        return self._launch(_lib.load().kx_adjoint, x, self.ni, "kx_adjoint")
+        return self._launch(x, self.ni, True)
 
     # several columns at once: the reference's matmat applies matvec column
     # by column (LO:436-460), and every column here is bitwise its matvec.
