@@ -442,6 +442,15 @@ int kx_eikonal(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, double hx, dou
                double hz, const double *slow, int32_t n, const int32_t *src, double *T,
                int32_t max_iter, int32_t order, int32_t *flag, int32_t *iters, void *stream);
 
+/* kx_eikonal with a workspace of at least kx_eikonal_work_bytes() (0 where
+ * none helps: 3D grids, and 2D grids whose shorter side exceeds 1024 cells):
+ * every sweep of a source then runs in one launch; the same times and rounds. */
+int64_t kx_eikonal_work_bytes(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, int32_t n);
+int kx_eikonal_ws(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, double hx, double hy,
+                  double hz, const double *slow, int32_t n, const int32_t *src, double *T,
+                  int32_t max_iter, int32_t order, int32_t *flag, int32_t *iters, void *work,
+                  int64_t work_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -29,7 +29,7 @@ EXPORTS = (
     "kx_cgls_scalar", "kx_lsqr_scalar", "kx_batch_dev_bytes", "kx_batch_build",
     "kx_batch_workspace_bytes", "kx_batch_forward", "kx_batch_adjoint",
     "kx_seg_workspace_bytes", "kx_seg_vec", "kx_seg_dot", "kx_cgls_scalar_batch",
-    "kx_eikonal", "kx_conv_rows", "kx_xcorr_rows", "kx_spread_models",
+    "kx_eikonal", "kx_eikonal_work_bytes", "kx_eikonal_ws", "kx_conv_rows", "kx_xcorr_rows", "kx_spread_models",
     "kx_gather_models", "kx_forward_noalloc",
 )
 
@@ -224,6 +224,9 @@ def _declare(L):
         "kx_cgls_scalar_batch": ([P, I32, P, P, I32, I32, P], ctypes.c_int),
         "kx_eikonal": ([I32, I32, I32, I32, D, D, D, P, I32, P, P, I32, I32, P,
                         ctypes.POINTER(I32), P], ctypes.c_int),  # iters: int32[2]
+        "kx_eikonal_work_bytes": ([I32, I32, I32, I32, I32], I64),
+        "kx_eikonal_ws": ([I32, I32, I32, I32, D, D, D, P, I32, P, P, I32, I32, P,
+                           ctypes.POINTER(I32), P, I64, P], ctypes.c_int),
     }
     for name, (args, res) in sig.items():
         f = getattr(L, name)

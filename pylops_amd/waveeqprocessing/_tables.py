@@ -104,10 +104,15 @@ def eikonal(pts, vel, origin, dsamp, dims, device, unit=False, max_iter=20, orde
     flag = torch.zeros(1, dtype=torch.int32, device=device)
     iters = (ctypes.c_int32 * 2)(0, 0)
     L = _lib.load()
-    rc = L.kx_eikonal(ndims, nx, ny, nz, hx, hy, hz, _lib.ptr(slow.contiguous()), n,
-                      _lib.ptr(srcd), _lib.ptr(out), max_iter, order, _lib.ptr(flag),
-                      iters, _lib.stream_ptr(device))
-    _lib.check(rc, "kx_eikonal")
+    slow = slow.contiguous()
+    # room for the sweeps of a 2D grid to run in one launch
+    work = torch.empty(L.kx_eikonal_work_bytes(ndims, nx, ny, nz, n), dtype=torch.uint8,
+                       device=device)
+    rc = L.kx_eikonal_ws(ndims, nx, ny, nz, hx, hy, hz, _lib.ptr(slow), n, _lib.ptr(srcd),
+                         _lib.ptr(out), max_iter, order, _lib.ptr(flag), iters,
+                         _lib.ptr(work) if work.numel() else None, work.numel(),
+                         _lib.stream_ptr(device))
+    _lib.check(rc, "kx_eikonal_ws")
     if not iters[1]:
         # an unconverged sweep leaves upper bounds, not first arrivals
         raise RuntimeError(
@@ -119,15 +124,19 @@ def eikonal(pts, vel, origin, dsamp, dims, device, unit=False, max_iter=20, orde
 def eikonal_tables(srcs, recs, vel, origin, dsamp, dims, device, distances, max_iter=20):
     """(trav_srcs, trav_recs, dist_srcs, dist_recs, grad_srcs, grad_recs) of
     the eikonal mode (K:609-657): first-arrival times from each source and
-    receiver cell, the unit-speed distances when ``distances`` (dynamic
-    amplitudes need them), and the traveltime gradients; ``max_iter`` sweep
-    rounds per phase at most (RuntimeError if they do not converge)."""
-    ts = eikonal(srcs, vel, origin, dsamp, dims, device, max_iter=max_iter)
-    tr = eikonal(recs, vel, origin, dsamp, dims, device, max_iter=max_iter)
-    ds = dr = None
-    if distances:
-        ds = eikonal(srcs, None, origin, dsamp, dims, device, unit=True, max_iter=max_iter)
-        dr = eikonal(recs, None, origin, dsamp, dims, device, unit=True, max_iter=max_iter)
+    receiver cell, and when ``distances`` (the dynamic weights need them) the
+    unit-speed distances and the traveltime gradients, None otherwise;
+    ``max_iter`` sweep rounds per phase at most (RuntimeError if they do not
+    converge)."""
+    # sources and receivers in one call: a table's sweeps are a chain of
+    # dependent steps, and every table has its own workgroup
+    pts, ns = np.hstack((srcs, recs)), np.asarray(srcs).shape[1]
+    t = eikonal(pts, vel, origin, dsamp, dims, device, max_iter=max_iter)
+    ts, tr = t[:, :ns], t[:, ns:]
+    if not distances:
+        return ts, tr, None, None, None, None
+    d = eikonal(pts, None, origin, dsamp, dims, device, unit=True, max_iter=max_iter)
+    ds, dr = d[:, :ns], d[:, ns:]
     return ts, tr, ds, dr, gradient(ts, dims, dsamp), gradient(tr, dims, dsamp)
 
 
