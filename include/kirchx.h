@@ -66,6 +66,16 @@ extern "C" {
 /* plan.dynamic value for dynamic plans whose aperture gates are all 0 */
 #define KX_DYNAMIC_NOGATE 2
 
+/* kx_plan.tabs: */
+/* every receiver table (off_r and, when dynamic, wp_r and wq_r) is followed in
+ * memory by its slot-ordered copy (kx_slot_table) */
+#define KX_TAB_SLOTS 1
+/* every sample of a group of 1, 2 or 4 tiles lies in the adjoint's staged
+ * windows (kx_table_fit) */
+#define KX_TAB_FIT1 2
+#define KX_TAB_FIT2 4
+#define KX_TAB_FIT4 8
+
 /* element types */
 #define KX_F32 0
 #define KX_F64 1
@@ -129,9 +139,7 @@ typedef struct kx_plan {
     int32_t gtiles; /* neighbouring image tiles per wave in the adjoint (1, 2
                        or 4; they share the staged trace windows),
                        0 = automatic */
-    int32_t slots;  /* 1: every receiver table (off_r and, when dynamic, wp_r
-                       and wq_r) is followed in memory by its slot-ordered
-                       copy (kx_slot_table); 0: it is not */
+    int32_t tabs;   /* what is known of the tables, KX_TAB_* bits (0: nothing) */
     double wtyp;  /* typical |weight| of one (point, trace) pair: 1 kinematic,
                      mean_s |(wp_s, wq_s)| * mean_r |(wp_r, wq_r)| over the
                      nonzero weights dynamic (0: taken as wamp).  A float32
@@ -170,11 +178,16 @@ int kx_tile_table(const kx_plan *geom, const double *tabT, int32_t n,
  * behind it: tab holds ntiles*n*64 elements of fmt (KX_F32 or KX_F16; offsets
  * or weights) and room for kx_slot_table_elems(geom, n) more.  The copy is
  * the order in which the forward's blocks of 8 and 16 receivers read the
- * table (plan.slots = 1): per tile and block of 16 receivers, chunks of 16
+ * table (KX_TAB_SLOTS): per tile and block of 16 receivers, chunks of 16
  * bytes of consecutive points of one receiver, so that the lanes of a wave
  * read contiguous memory.  (No reference counterpart: device layout.) */
 int64_t kx_slot_table_elems(const kx_plan *geom, int32_t n);
 int kx_slot_table(const kx_plan *geom, int32_t n, int32_t fmt, void *tab, void *stream);
+
+/* Which KX_TAB_FIT* bits hold for the plan's traveltime tables (written to
+ * *tabs on the host): with them the adjoint needs no test for samples outside
+ * its windows.  scratch: 64 bytes of device memory.  Synchronises the stream. */
+int kx_table_fit(const kx_plan *p, void *scratch, int32_t *tabs, void *stream);
 
 /* The engine kernels alone.
  * kx_spread: traces[ns*nr][nt] = sum over image points of m spread at the

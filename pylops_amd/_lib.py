@@ -18,11 +18,12 @@ KX_F32, KX_F64, KX_F16 = 0, 1, 2
 KX_ORDER_AUTO, KX_ORDER_NATURAL, KX_ORDER_ROTATED = 0, 1, 2
 KX_SIDE_AUTO, KX_SIDE_RECEIVERS, KX_SIDE_SOURCES = 0, 1, 2
 KX_DYNAMIC_NOGATE = 2
+KX_TAB_SLOTS, KX_TAB_FIT1, KX_TAB_FIT2, KX_TAB_FIT4 = 1, 2, 4, 8
 KX_EINVAL, KX_ESHAPE, KX_ETYPE, KX_EABI, KX_ELDS = -1, -2, -3, -4, -5
 
 EXPORTS = (
     "kx_version", "kx_last_error", "kx_workspace_bytes", "kx_encode_table",
-    "kx_tile_table", "kx_slot_table_elems", "kx_slot_table", "kx_spread",
+    "kx_tile_table", "kx_slot_table_elems", "kx_slot_table", "kx_table_fit", "kx_spread",
     "kx_gather", "kx_conv", "kx_forward", "kx_forward_work_bytes", "kx_forward_ws",
     "kx_adjoint", "kx_reduce_workspace_bytes", "kx_dot",
     "kx_solver_workspace_bytes", "kx_vec", "kx_dot_dev", "kx_lsqr_xw",
@@ -130,7 +131,7 @@ class KxPlan(ctypes.Structure):
         ("gsplit", ctypes.c_int32),
         ("sside", ctypes.c_int32),
         ("gtiles", ctypes.c_int32),
-        ("slots", ctypes.c_int32),
+        ("tabs", ctypes.c_int32),
         ("wtyp", ctypes.c_double),
     ]
 
@@ -193,6 +194,7 @@ def _declare(L):
         "kx_tile_table": ([PP, P, I32, I32, P, P], ctypes.c_int),
         "kx_slot_table_elems": ([PP, I32], I64),
         "kx_slot_table": ([PP, I32, I32, P, P], ctypes.c_int),
+        "kx_table_fit": ([PP, P, ctypes.POINTER(I32), P], ctypes.c_int),
         "kx_spread": ([PP, P, P, P], ctypes.c_int),
         "kx_gather": ([PP, P, P, P], ctypes.c_int),
         "kx_spread_models": ([PP, P, P, I32, P], ctypes.c_int),

@@ -87,6 +87,7 @@ extern "C" __attribute__((visibility("hidden"))) int kx_plan_check(const kx_plan
 extern "C" const char *kx_last_error(void) { return g_err; }
 
 #include "kx_device.h"
+#include "kx_fit.h"
 
 // ---------------------------------------------------------------------------
 // single-problem kernels
@@ -211,6 +212,73 @@ __global__ __launch_bounds__(kBlock) void slot_kernel(const TT *__restrict__ tab
     const int p = ((w >> 4) & 3) * 16 + (w >> 6) * CH;
     reinterpret_cast<VecN<TT, CH> *>(out)[i] =
         *reinterpret_cast<const VecN<TT, CH> *>(tab + (t * n + j) * kWave + p);
+}
+
+// Largest |base + offset - mean base| over groups of 1, 2 and 4 tiles of one
+// side's table (out[0..2], float bits, all positive): how far a sample can
+// lie from the middle of its group's window on that side's account.  One wave
+// per (group of 4, entry) pair, striding; entries no sample can take have
+// offsets far outside any window, and bases beyond 2^24 count as such.
+template <typename TT>
+__global__ __launch_bounds__(kBlock) void fit_kernel(KArgs a, const TT *__restrict__ off,
+                                                     const int *__restrict__ base, int n,
+                                                     unsigned *__restrict__ out)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t nw = (int64_t)gridDim.x * (kBlock / kWave), total = (int64_t)a.ngroups * n;
+    float e1 = 0.f, e2 = 0.f, e4 = 0.f;
+    for (int64_t w = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; w < total;
+         w += nw) {
+        const int g = (int)(w / n), r = (int)(w % n);
+        const int tzi = g % a.ntz, rest = g / a.ntz;
+        const int x0 = (rest % a.ngx) * a.gx, y0 = (rest / a.ngx) * a.gy;
+        int b[4];
+        float o[4];
+        bool ok[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int x = x0 + j % a.gx, y = y0 + j / a.gx;
+            ok[j] = x < a.ntx && y < a.nty;
+            const size_t at = ((size_t)(tzi + a.ntz * (ok[j] ? x + a.ntx * y : x0 + a.ntx * y0))) * n + r;
+            b[j] = base[at];
+            o[j] = (float)ld_off(off + at * kWave + lane);
+            if (abs(b[j]) >= (1 << 24) || !(fabsf(o[j]) < 1e30f))  // NaN too
+                o[j] = 1e30f;
+            e1 = fmaxf(e1, fabsf(o[j]));
+        }
+        const int m4 = (b[0] + b[1] + b[2] + b[3]) >> 2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            e4 = fmaxf(e4, fabsf((float)(b[j] - m4) + o[j]));
+            // pairs (0, 1) and (2, 3); a second tile past the edge repeats
+            // the first
+            const int j0 = j & 2, j1 = ok[j0 + 1] ? j0 + 1 : j0;
+            const int m2 = (b[j0] + b[j1]) >> 1;
+            if (ok[j0] && ok[j])
+                e2 = fmaxf(e2, fabsf((float)(b[j] - m2) + o[j]));
+        }
+    }
+#pragma unroll
+    for (int s = kWave / 2; s >= 1; s >>= 1) {
+        e1 = fmaxf(e1, __shfl_xor(e1, s, kWave));
+        e2 = fmaxf(e2, __shfl_xor(e2, s, kWave));
+        e4 = fmaxf(e4, __shfl_xor(e4, s, kWave));
+    }
+    if (lane == 0) {
+        atomicMax(&out[0], __float_as_uint(e1));
+        atomicMax(&out[1], __float_as_uint(e2));
+        atomicMax(&out[2], __float_as_uint(e4));
+    }
+}
+
+template <typename TT>
+void launch_fit(const KArgs &a, const void *off, const int *base, int n, unsigned *out,
+                hipStream_t st)
+{
+    const int64_t waves = (int64_t)a.ngroups * n;
+    const int nblk = (int)std::min<int64_t>(4096, (waves + 3) / 4);
+    hipLaunchKernelGGL(fit_kernel<TT>, dim3(nblk), dim3(kBlock), 0, st, a,
+                       reinterpret_cast<const TT *>(off), base, n, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -413,6 +481,40 @@ extern "C" int kx_slot_table(const kx_plan *geom, int32_t n, int32_t fmt, void *
                            reinterpret_cast<const __half *>(tab), n, nchunk,
                            reinterpret_cast<__half *>(tab) + plain);
     KX_LAUNCHED("slot_table");
+    return KX_OK;
+}
+
+extern "C" int kx_table_fit(const kx_plan *p, void *scratch, int32_t *tabs, void *stream)
+{
+    int rc = check_plan(p);
+    if (rc)
+        return rc;
+    if (!scratch || !tabs)
+        return kx_fail(KX_EINVAL, "table_fit: NULL buffer");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    unsigned *out = static_cast<unsigned *>(scratch);
+    KArgs a = make_args(p);
+    set_tile_groups(a, 4);
+    KX_HIP(hipMemsetAsync(out, 0, 64, st));
+    if (p->dtype == KX_F64) {
+        launch_fit<double>(a, p->off_s, p->base_s, p->ns, out, st);
+        launch_fit<double>(a, p->off_r, p->base_r, p->nr, out + 4, st);
+    } else {
+        launch_fit<float>(a, p->off_s, p->base_s, p->ns, out, st);
+        if (p->tab_fmt == KX_F16)
+            launch_fit<__half>(a, p->off_r, p->base_r, p->nr, out + 4, st);
+        else
+            launch_fit<float>(a, p->off_r, p->base_r, p->nr, out + 4, st);
+    }
+    KX_LAUNCHED("table_fit");
+    float e[8];
+    KX_HIP(hipMemcpyAsync(e, out, sizeof(e), hipMemcpyDeviceToHost, st));
+    KX_HIP(hipStreamSynchronize(st));
+    *tabs = 0;
+    const int bit[3] = {KX_TAB_FIT1, KX_TAB_FIT2, KX_TAB_FIT4};
+    for (int k = 0; k < 3; ++k)
+        if (e[k] + e[4 + k] <= kFitBound)
+            *tabs |= bit[k];
     return KX_OK;
 }
 

@@ -79,6 +79,18 @@ __device__ __forceinline__ float ld_off(const float *p) { return *p; }
 __device__ __forceinline__ float ld_off(const __half *p) { return __half2float(*p); }
 __device__ __forceinline__ double ld_off(const double *p) { return *p; }
 
+// A wave-uniform global pointer kept in scalar registers: loads through it
+// with a 32-bit lane offset need no vector arithmetic for their addresses
+// (the compiler otherwise keeps pointer + lane in vector registers and adds
+// the tile's offset to each).
+template <typename T> using GlobalPtr = const __attribute__((address_space(1))) T *;
+template <typename T> __device__ __forceinline__ GlobalPtr<T> scalar_ptr(const T *p)
+{
+    GlobalPtr<T> g = (GlobalPtr<T>)p;
+    asm volatile("" : "+s"(g));
+    return g;
+}
+
 // Hardware dispatches workgroup b to XCD (b mod 8).  Renumber so that each
 // XCD receives a contiguous range of logical blocks: neighbouring image
 // tiles (gather) or the same receiver block (spread) then share one L2.
@@ -97,6 +109,7 @@ struct KArgs {
     int ntz, ntx, nty;
     int ntiles;
     int rblock;
+    int tabs;  // kx_plan.tabs
     // adjoint tile groups: gx x gy tiles, ngx x ngy groups per z row,
     // ngroups in all (set_tile_groups; 1 x 1 by default)
     int gx, gy, ngx, ngy, ngroups;
@@ -132,6 +145,7 @@ inline KArgs make_args(const kx_plan *p)
     a.nty = p->nty;
     a.ntiles = (int)p->ntiles;
     a.rblock = p->rblock;
+    a.tabs = p->tabs;
     a.gx = a.gy = 1;
     a.ngx = p->ntx;
     a.ngy = p->nty;
@@ -206,7 +220,7 @@ __device__ __forceinline__ int64_t point_index(const KArgs &a, const TilePoint &
 // ---------------------------------------------------------------------------
 // slot-ordered receiver tables
 // ---------------------------------------------------------------------------
-// The copy behind a receiver table (kx_plan.slots): per tile and block of
+// The copy behind a receiver table (KX_TAB_SLOTS): per tile and block of
 // kSlotBlock receivers, 16-byte chunks of consecutive points of one receiver,
 // chunk c of row group q (points 16 q + SlotChunkLen c ...) of receiver j at
 // chunk index (c 4 + q) 16 + j: lane 16 q + j of a wave reads chunk c of its
@@ -1175,6 +1189,13 @@ template <int N> struct IntC {
     static constexpr int value = N;
 };
 
+// weight of a pair in the adjoint (fused the same way in every kernel, so
+// that their images are bitwise alike; so is its product with the sample)
+template <typename TD> __device__ __forceinline__ TD pair_weight(TD ps, TD pr, TD qs, TD qr)
+{
+    return fma(ps, pr, qs * qr);
+}
+
 template <int NP> struct Log2 {
     static constexpr int v = NP >= 4 ? 2 : (NP >= 2 ? 1 : 0);
 };
@@ -1195,6 +1216,53 @@ inline void set_tile_groups(KArgs &a, int np)
     a.ngx = (a.ntx + a.gx - 1) / a.gx;
     a.ngy = (a.nty + a.gy - 1) / a.gy;
     a.ngroups = a.ntz * a.ngx * a.ngy;
+}
+
+// The end of a gather workgroup: with P > 1 the partial sums of a group's
+// points, one part per wave, are added in part order through lds; part 0
+// writes the image.
+template <typename TD, int P, int NP, int K>
+__device__ __forceinline__ void gather_store(const KArgs &a, TD (&acc)[K][NP], void *lds,
+                                             TD *__restrict__ m, int64_t mstride, int part,
+                                             int wave, int lane, bool active,
+                                             const bool (&tok)[NP], const TilePoint (&pt)[NP])
+{
+    constexpr int NG = kGatherWaves / P;
+    if constexpr (P > 1) {
+        // the partial sums of a group's points, added in part order
+        __syncthreads();
+        TD *red = reinterpret_cast<TD *>(lds);
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int j = 0; j < NP; ++j)
+                red[(k * NP + j) * kGatherBlock + threadIdx.x] = acc[k][j];
+        __syncthreads();
+        if (part == 0) {
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+#pragma unroll
+                for (int j = 0; j < NP; ++j) {
+                    acc[k][j] = TD(0);
+#pragma unroll
+                    for (int q = 0; q < P; ++q)
+                        acc[k][j] += red[(k * NP + j) * kGatherBlock + (q * NG + wave) * kWave + lane];
+                }
+        }
+    }
+    if (part == 0 && active) {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            if (tok[j] && pt[j].valid) {
+                const int64_t pi = point_index(a, pt[j]);
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    m[k * mstride + pi] = acc[k][j];
+            }
+        }
+    }
+    if constexpr (P > 1)
+        __syncthreads();  // the partial sums are read before a next item stages
 }
 
 // K > 1: the data of K models (model k at d + k*dstride, its image at
@@ -1424,7 +1492,7 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
                     const unsigned kc = min(kk, (unsigned)(kWin - 1));
                     TD wgt = TD(1);
                     if constexpr (DYN) {
-                        wgt = ps[i][j] * pr[j] + qs[i][j] * qr[j];
+                        wgt = pair_weight(ps[i][j], pr[j], qs[i][j], qr[j]);
                         if (GATE && pt[j].iz < izr[i])
                             wgt = TD(0);
                     }
@@ -1432,9 +1500,7 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
                     for (int k = 0; k < K; ++k) {
                         const TP q = w[k][i][kc];
                         TD v = fma((TD)f, q.v[1], q.v[0]);
-                        if constexpr (DYN)
-                            v *= wgt;
-                        acc[k][j] += v;
+                        acc[k][j] = DYN ? fma(v, wgt, acc[k][j]) : acc[k][j] + v;
                     }
                 }
             }
@@ -1459,7 +1525,7 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
                             if ((unsigned)it < ntm1) {
                                 TD wgt = TD(1);
                                 if constexpr (DYN) {
-                                    wgt = ps[i][j] * pr[j] + qs[i][j] * qr[j];
+                                    wgt = pair_weight(ps[i][j], pr[j], qs[i][j], qr[j]);
                                     if (GATE && pt[j].iz < izr[i])
                                         wgt = TD(0);
                                 }
@@ -1468,9 +1534,7 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
                                     const TD *q = dblk + k * dstride + (soff[i] + r * a.nt + it);
                                     const TD g0 = q[0], g1 = q[1];
                                     TD v = fma((TD)f, g1 - g0, g0);
-                                    if constexpr (DYN)
-                                        v *= wgt;
-                                    acc[k][j] += v;
+                                    acc[k][j] = DYN ? fma(v, wgt, acc[k][j]) : acc[k][j] + v;
                                 }
                             }
                         }
@@ -1490,41 +1554,8 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
                 source_block(IntC<(JW > 1 ? JW / 2 : 1)>{}, s0);
         }
     }
-    if constexpr (P > 1) {
-        // the partial sums of a group's points, added in part order
-        __syncthreads();
-        TD *red = reinterpret_cast<TD *>(&win[0][0][0][0]);
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-#pragma unroll
-            for (int j = 0; j < NP; ++j)
-                red[(k * NP + j) * kGatherBlock + threadIdx.x] = acc[k][j];
-        __syncthreads();
-        if (part == 0) {
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-#pragma unroll
-                for (int j = 0; j < NP; ++j) {
-                    acc[k][j] = TD(0);
-#pragma unroll
-                    for (int q = 0; q < P; ++q)
-                        acc[k][j] += red[(k * NP + j) * kGatherBlock + (q * NG + wave) * kWave + lane];
-                }
-        }
-    }
-    if (part == 0 && active) {
-#pragma unroll
-        for (int j = 0; j < NP; ++j) {
-            if (tok[j] && pt[j].valid) {
-                const int64_t pi = point_index(a, pt[j]);
-#pragma unroll
-                for (int k = 0; k < K; ++k)
-                    m[k * mstride + pi] = acc[k][j];
-            }
-        }
-    }
-    if constexpr (P > 1)
-        __syncthreads();  // the partial sums are read before a next item stages
+    gather_store<TD, P, NP, K>(a, acc, &win[0][0][0][0], m, mstride, part, wave, lane, active, tok,
+                               pt);
 }
 
 // ---------------------------------------------------------------------------

@@ -9,6 +9,7 @@
 
 #include "kx_internal.h"
 #include "kx_device.h"
+#include "kx_fit.h"
 
 namespace {
 
@@ -23,6 +24,33 @@ __global__ __launch_bounds__(kGatherBlock) void gather_kernel(KArgs a, const TD 
 {
     gather_tiles<TD, TT, DYN, NEG, JW, P, NP, K, GATE>(a, d, m, xcd_remap(blockIdx.x, gridDim.x),
                                                        dstride, mstride);
+}
+
+int device_cus()
+{
+    int cus = 256, dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        (void)hipGetLastError();
+        cus = 256;
+    }
+    return cus;
+}
+
+// waves per SIMD asked of the compiler: with two tiles a dynamic group takes
+// 91 vector registers, five waves; six (80 registers, a few words of scratch
+// outside the receiver loop) measured 1.88 -> 1.72 ms on 2D 601x300
+template <typename TD, bool DYN, int NP, int K> struct FitWaves {
+    static constexpr int v = (DYN && NP == 2 && K == 1 && sizeof(TD) == 4) ? 6 : 1;
+};
+
+// the same for plans whose samples all lie in their windows
+template <typename TD, typename TT, bool DYN, int JW, int P, int NP, int K, bool GATE>
+__global__ __launch_bounds__(kGatherBlock, (FitWaves<TD, DYN, NP, K>::v)) void gather_fit_kernel(
+    KArgs a, const TD *__restrict__ d, TD *__restrict__ m, int64_t dstride, int64_t mstride)
+{
+    gather_fit<TD, TT, DYN, JW, P, NP, K, GATE>(a, d, m, xcd_remap(blockIdx.x, gridDim.x), dstride,
+                                                mstride);
 }
 
 // sources per wave and pass (measured): every pass re-reads the receiver
@@ -42,6 +70,24 @@ int launch_gather_p(KArgs a, const void *d, int64_t dstride, void *m, int64_t ms
         return kx_failf(KX_ESHAPE, "gather: %d sources x nr x nt exceeds 2^31 samples", JW * P);
     set_tile_groups(a, NP);
     const int nblk = (a.ngroups + NG - 1) / NG;
+    if constexpr (!NEG) {
+        // Plans with a sample outside the windows, or whose block of sources
+        // is too large for 31-bit byte offsets, and negative times take the
+        // general kernel.  So do launches of less than a wave per SIMD, which
+        // wait for memory, not for instructions: the adjoint of a 101x100
+        // grid, 11 x 51 traces, 27.5 us there and 28.6 here (a dynamic
+        // 121x81 gather 37.8 and 38.8); 201x101, 20 x 51 traces, the gather
+        // alone 37.9 and 31.8, 301x201 dynamic 117 and 90.
+        constexpr int fit = NP == 4 ? KX_TAB_FIT4 : (NP == 2 ? KX_TAB_FIT2 : KX_TAB_FIT1);
+        if ((a.tabs & fit) && nblk >= device_cus() &&
+            (int64_t)JW * P * a.nr * a.nt * (int64_t)sizeof(TD) < ((int64_t)1 << 30)) {
+            hipLaunchKernelGGL((gather_fit_kernel<TD, TT, DYN, JW, P, NP, K, GATE>), dim3(nblk),
+                               dim3(kGatherBlock), 0, st, a, reinterpret_cast<const TD *>(d),
+                               reinterpret_cast<TD *>(m), dstride, mstride);
+            KX_LAUNCHED("gather");
+            return KX_OK;
+        }
+    }
     hipLaunchKernelGGL((gather_kernel<TD, TT, DYN, NEG, JW, P, NP, K, GATE>), dim3(nblk),
                        dim3(kGatherBlock), 0, st, a, reinterpret_cast<const TD *>(d),
                        reinterpret_cast<TD *>(m), dstride, mstride);
@@ -56,17 +102,6 @@ int launch_gather_p(KArgs a, const void *d, int64_t dstride, void *m, int64_t ms
 // give every CU kGatherFill waves (measured: 2D 601x300 dynamic 2 x 4,
 // 2.5 ms; 3D 128x128x120 4 x 4, 8.8 ms).
 constexpr int kGatherFill = 20;
-
-int device_cus()
-{
-    int cus = 256, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-        (void)hipGetLastError();
-        cus = 256;
-    }
-    return cus;
-}
 
 int gather_jw(bool dyn, int np, int k) { return (dyn && np == 1 && k == 1) ? 8 : 4; }
 

@@ -111,17 +111,6 @@ struct SlotPoint {
     int iz;      // depth index of the lane's point
 };
 
-// A wave-uniform global pointer kept in scalar registers: loads through it
-// with a 32-bit lane offset need no vector arithmetic for their addresses
-// (the compiler otherwise keeps pointer + lane in vector registers and adds
-// the tile's offset to each).
-template <typename T> using GlobalPtr = const __attribute__((address_space(1))) T *;
-template <typename T> __device__ __forceinline__ GlobalPtr<T> scalar_ptr(const T *p)
-{
-    GlobalPtr<T> g = (GlobalPtr<T>)p;
-    asm volatile("" : "+s"(g));
-    return g;
-}
 typedef unsigned Words4 __attribute__((ext_vector_type(4)));
 
 // What a lane needs to know to load its tiles.

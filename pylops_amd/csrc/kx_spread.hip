@@ -293,7 +293,7 @@ struct SlotsShape {
 SlotsShape pick_slots(const kx_plan *p, int nh, int64_t work_bytes)
 {
     SlotsShape best{0, 0, 0, 1, 0, 0};
-    if (!p->slots || p->dtype != KX_F32 || p->sside == KX_SIDE_SOURCES)
+    if (!(p->tabs & KX_TAB_SLOTS) || p->dtype != KX_F32 || p->sside == KX_SIDE_SOURCES)
         return best;
     const int cus = device_cus();
     const bool half = p->tab_fmt == KX_F16;

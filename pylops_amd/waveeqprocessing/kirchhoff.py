@@ -448,7 +448,7 @@ class Kirchhoff(LinearOperator):
             plan.dynamic = _lib.KX_DYNAMIC_NOGATE
         plan.ns, plan.nr, plan.nt = ns, nr, self.nt
         plan.neg_trav = int(neg)
-        plan.slots = int(slots)
+        plan.tabs = _lib.KX_TAB_SLOTS if slots else 0
         plan.rblock = self.rblock
         plan.sorder = self.sorder
         plan.sside = self.sside
@@ -457,6 +457,11 @@ class Kirchhoff(LinearOperator):
         plan.nh = keep["h"].numel()
         for k, v in keep.items():
             setattr(plan, k, v.data_ptr())
+        fit = ctypes.c_int32(0)
+        _lib.check(_lib.load().kx_table_fit(ctypes.byref(plan), _lib.ptr(keep["aux"]),
+                                            ctypes.byref(fit), _lib.stream_ptr(dev)),
+                   "kx_table_fit")
+        plan.tabs |= fit.value
         object.__setattr__(self, "_dev_tables", keep)
         object.__setattr__(self, "_plan", plan)
         object.__setattr__(self, "_ws_key", None)
