@@ -377,7 +377,10 @@ int kx_lsqr_scalar(double *sc, double *cost, int32_t phase, void *stream);
 typedef struct kx_batch {
     int32_t abi_version;
     int32_t nprob;
-    int32_t dtype, tab_fmt, dynamic, neg_trav;
+    int32_t dtype, tab_fmt, dynamic;
+    int32_t neg_trav;          /* 1: negative times; -1: none, and the samples of some
+                                  problems lie in the adjoint's windows (KX_TAB_FIT*);
+                                  0: neither */
     int32_t rblock;            /* forward receivers per workgroup (all problems) */
     int32_t sorder;            /* forward lane order (all problems) */
     int32_t gsplit;            /* adjoint waves per tile (all problems) */

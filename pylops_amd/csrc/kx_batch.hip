@@ -45,6 +45,7 @@ extern "C" int kx_solver_fail(int code, const char *msg);
 extern "C" int kx_plan_check(const kx_plan *p);
 
 #include "kx_device.h"
+#include "kx_fit.h"
 
 namespace {
 
@@ -165,8 +166,16 @@ __global__ __launch_bounds__(kSpreadBlock) void batch_spread_kernel(
     launch_done(ctr);
 }
 
-template <typename TD, typename TT, bool DYN, bool NEG, int JW, int P, int NP>
-__global__ __launch_bounds__(kGatherBlock) void batch_gather_kernel(
+// times of a batch (kx_batch.neg_trav): negative ones; none, and the samples
+// of some problems all in their windows (KX_TAB_FIT*), which take the kernel
+// of kx_fit.h (chosen per item; 24 problems up to 512x256 with float16
+// tables, 21 of which fit: 1.53 -> 1.27 ms); neither
+constexpr int kTimesFit = -1, kTimesAny = 0, kTimesNeg = 1;
+
+template <typename TD, typename TT, bool DYN, int TIMES, int JW, int P, int NP>
+__global__ __launch_bounds__(kGatherBlock,
+                             (TIMES == kTimesFit ? FitWaves<TD, DYN, NP, 1>::v : 1)) void
+batch_gather_kernel(
     const BatchProb *__restrict__ probs, const GatherItem *__restrict__ items, unsigned *ctr,
     const int *__restrict__ qoff, const TD *__restrict__ d, TD *__restrict__ m)
 {
@@ -178,8 +187,14 @@ __global__ __launch_bounds__(kGatherBlock) void batch_gather_kernel(
             break;
         const GatherItem w = items[it];
         const KArgs a = probs[w.p].a;
-        gather_tiles<TD, TT, DYN, NEG, JW, P, NP>(a, d + probs[w.p].doff, m + probs[w.p].moff,
-                                                  w.L);
+        const TD *dp = d + probs[w.p].doff;
+        TD *mp = m + probs[w.p].moff;
+        if constexpr (TIMES == kTimesFit)
+            if (a.tabs & (NP == 2 ? KX_TAB_FIT2 : KX_TAB_FIT1)) {
+                gather_fit<TD, TT, DYN, JW, P, NP, 1, true>(a, dp, mp, w.L, 0, 0);
+                continue;
+            }
+        gather_tiles<TD, TT, DYN, TIMES == kTimesNeg, JW, P, NP>(a, dp, mp, w.L);
     }
     launch_done(ctr);
 }
@@ -308,24 +323,24 @@ template <bool DYN, int NP> struct BatchJW {
 };
 int batch_jw(bool dyn, int np) { return (dyn && np == 1) ? 8 : 4; }
 
-template <typename TD, typename TT, bool DYN, bool NEG, int NP>
+template <typename TD, typename TT, bool DYN, int TIMES, int NP>
 const void *bgather_fn_np(int P)
 {
     constexpr int JW = BatchJW<DYN, NP>::v;
     switch (P) {
     case 1:
-        return reinterpret_cast<const void *>(&batch_gather_kernel<TD, TT, DYN, NEG, JW, 1, NP>);
+        return reinterpret_cast<const void *>(&batch_gather_kernel<TD, TT, DYN, TIMES, JW, 1, NP>);
     case 2:
-        return reinterpret_cast<const void *>(&batch_gather_kernel<TD, TT, DYN, NEG, JW, 2, NP>);
+        return reinterpret_cast<const void *>(&batch_gather_kernel<TD, TT, DYN, TIMES, JW, 2, NP>);
     default:
-        return reinterpret_cast<const void *>(&batch_gather_kernel<TD, TT, DYN, NEG, JW, 4, NP>);
+        return reinterpret_cast<const void *>(&batch_gather_kernel<TD, TT, DYN, TIMES, JW, 4, NP>);
     }
 }
 
-template <typename TD, typename TT, bool DYN, bool NEG>
+template <typename TD, typename TT, bool DYN, int TIMES>
 const void *bgather_fn(int P, int np)
 {
-    return np == 2 ? bgather_fn_np<TD, TT, DYN, NEG, 2>(P) : bgather_fn_np<TD, TT, DYN, NEG, 1>(P);
+    return np == 2 ? bgather_fn_np<TD, TT, DYN, TIMES, 2>(P) : bgather_fn_np<TD, TT, DYN, TIMES, 1>(P);
 }
 
 // Resident workgroups of a kernel per CU; without a device, the LDS and
@@ -350,7 +365,7 @@ size_t spread_lds(int rb, int nt) { return (size_t)rb * trace_stride(nt) * 8; }
 // Kernel entry points of a batch, by its element and table types.
 struct Fns {
     const void *(*spread)(int rb, bool rot, bool dyn, bool neg);
-    const void *(*gather)(int P, int np, bool dyn, bool neg);
+    const void *(*gather)(int P, int np, bool dyn, int times);
 };
 
 template <typename TD, typename TT>
@@ -367,12 +382,18 @@ const void *spread_of(int rb, bool rot, bool dyn, bool neg)
                       : bspread_fn<TD, TT, false, false, false>(rb));
 }
 
-template <typename TD, typename TT>
-const void *gather_of(int P, int np, bool dyn, bool neg)
+template <typename TD, typename TT, int TIMES>
+const void *gather_of_times(int P, int np, bool dyn)
 {
-    if (dyn)
-        return neg ? bgather_fn<TD, TT, true, true>(P, np) : bgather_fn<TD, TT, true, false>(P, np);
-    return neg ? bgather_fn<TD, TT, false, true>(P, np) : bgather_fn<TD, TT, false, false>(P, np);
+    return dyn ? bgather_fn<TD, TT, true, TIMES>(P, np) : bgather_fn<TD, TT, false, TIMES>(P, np);
+}
+
+template <typename TD, typename TT>
+const void *gather_of(int P, int np, bool dyn, int times)
+{
+    return times == kTimesFit   ? gather_of_times<TD, TT, kTimesFit>(P, np, dyn)
+           : times == kTimesNeg ? gather_of_times<TD, TT, kTimesNeg>(P, np, dyn)
+                                : gather_of_times<TD, TT, kTimesAny>(P, np, dyn);
 }
 
 Fns fns_of(int dtype, int tab_fmt)
@@ -640,24 +661,24 @@ int launch_bspread_d(const kx_batch *b, const View &v, const void *m, void *y, h
 {
     const bool rot = b->sorder == KX_ORDER_ROTATED;
     if (b->dynamic) {
-        if (b->neg_trav)
+        if (b->neg_trav == kTimesNeg)
             return rot ? launch_bspread_rb<TD, TT, true, true, true>(b, v, m, y, st)
                        : launch_bspread_rb<TD, TT, true, true, false>(b, v, m, y, st);
         return rot ? launch_bspread_rb<TD, TT, true, false, true>(b, v, m, y, st)
                    : launch_bspread_rb<TD, TT, true, false, false>(b, v, m, y, st);
     }
-    if (b->neg_trav)
+    if (b->neg_trav == kTimesNeg)
         return rot ? launch_bspread_rb<TD, TT, false, true, true>(b, v, m, y, st)
                    : launch_bspread_rb<TD, TT, false, true, false>(b, v, m, y, st);
     return rot ? launch_bspread_rb<TD, TT, false, false, true>(b, v, m, y, st)
                : launch_bspread_rb<TD, TT, false, false, false>(b, v, m, y, st);
 }
 
-template <typename TD, typename TT, bool DYN, bool NEG, int P, int NP>
+template <typename TD, typename TT, bool DYN, int TIMES, int P, int NP>
 int launch_bgather(const kx_batch *b, const View &v, const void *d, void *m, hipStream_t st)
 {
     constexpr int JW = BatchJW<DYN, NP>::v;
-    hipLaunchKernelGGL((batch_gather_kernel<TD, TT, DYN, NEG, JW, P, NP>), dim3(b->grid_gather),
+    hipLaunchKernelGGL((batch_gather_kernel<TD, TT, DYN, TIMES, JW, P, NP>), dim3(b->grid_gather),
                        dim3(kGatherBlock), 0, st, v.probs, v.gitems, v.ctr + kGatherQ,
                        v.ctr_const + kQoff + 16, reinterpret_cast<const TD *>(d),
                        reinterpret_cast<TD *>(m));
@@ -665,34 +686,39 @@ int launch_bgather(const kx_batch *b, const View &v, const void *d, void *m, hip
     return KX_OK;
 }
 
-template <typename TD, typename TT, bool DYN, bool NEG, int NP>
+template <typename TD, typename TT, bool DYN, int TIMES, int NP>
 int launch_bgather_np(const kx_batch *b, const View &v, const void *d, void *m, hipStream_t st)
 {
     switch (b->gsplit) {
     case 1:
-        return launch_bgather<TD, TT, DYN, NEG, 1, NP>(b, v, d, m, st);
+        return launch_bgather<TD, TT, DYN, TIMES, 1, NP>(b, v, d, m, st);
     case 2:
-        return launch_bgather<TD, TT, DYN, NEG, 2, NP>(b, v, d, m, st);
+        return launch_bgather<TD, TT, DYN, TIMES, 2, NP>(b, v, d, m, st);
     default:
-        return launch_bgather<TD, TT, DYN, NEG, 4, NP>(b, v, d, m, st);
+        return launch_bgather<TD, TT, DYN, TIMES, 4, NP>(b, v, d, m, st);
     }
 }
 
-template <typename TD, typename TT, bool DYN, bool NEG>
+template <typename TD, typename TT, bool DYN, int TIMES>
 int launch_bgather_p(const kx_batch *b, const View &v, const void *d, void *m, hipStream_t st)
 {
-    return b->gtiles == 2 ? launch_bgather_np<TD, TT, DYN, NEG, 2>(b, v, d, m, st)
-                          : launch_bgather_np<TD, TT, DYN, NEG, 1>(b, v, d, m, st);
+    return b->gtiles == 2 ? launch_bgather_np<TD, TT, DYN, TIMES, 2>(b, v, d, m, st)
+                          : launch_bgather_np<TD, TT, DYN, TIMES, 1>(b, v, d, m, st);
+}
+
+template <typename TD, typename TT, int TIMES>
+int launch_bgather_t(const kx_batch *b, const View &v, const void *d, void *m, hipStream_t st)
+{
+    return b->dynamic ? launch_bgather_p<TD, TT, true, TIMES>(b, v, d, m, st)
+                      : launch_bgather_p<TD, TT, false, TIMES>(b, v, d, m, st);
 }
 
 template <typename TD, typename TT>
 int launch_bgather_d(const kx_batch *b, const View &v, const void *d, void *m, hipStream_t st)
 {
-    if (b->dynamic)
-        return b->neg_trav ? launch_bgather_p<TD, TT, true, true>(b, v, d, m, st)
-                           : launch_bgather_p<TD, TT, true, false>(b, v, d, m, st);
-    return b->neg_trav ? launch_bgather_p<TD, TT, false, true>(b, v, d, m, st)
-                       : launch_bgather_p<TD, TT, false, false>(b, v, d, m, st);
+    return b->neg_trav == kTimesFit   ? launch_bgather_t<TD, TT, kTimesFit>(b, v, d, m, st)
+           : b->neg_trav == kTimesNeg ? launch_bgather_t<TD, TT, kTimesNeg>(b, v, d, m, st)
+                                      : launch_bgather_t<TD, TT, kTimesAny>(b, v, d, m, st);
 }
 
 int launch_bconv(const kx_batch *b, const View &v, const void *x, void *y, int adjoint,
@@ -746,6 +772,7 @@ extern "C" int kx_batch_build(kx_batch *b, const kx_plan *plans, int32_t nprob, 
     std::vector<int64_t> cprefix(nprob + 1, 0);
     int64_t moff = 0, doff = 0;
     int nt_max = 0, nh_max = 0;
+    int times = q.neg_trav ? kTimesNeg : kTimesAny;
     for (int p = 0; p < nprob; ++p) {
         const kx_plan &a = plans[p];
         if ((int64_t)JW * c.P * a.nr * a.nt >= ((int64_t)1 << 31))
@@ -755,6 +782,12 @@ extern "C" int kx_batch_build(kx_batch *b, const kx_plan *plans, int32_t nprob, 
         B.a = make_args(&a);
         B.a.rblock = c.rb;
         set_tile_groups(B.a, c.np);
+        // (the windowed kernel addresses a block of sources in 31-bit bytes)
+        if ((int64_t)batch_jw(q.dynamic, c.np) * c.P * a.nr * a.nt * dsize(q.dtype) >=
+            ((int64_t)1 << 30))
+            B.a.tabs = 0;
+        if (!q.neg_trav && (B.a.tabs & (c.np == 2 ? KX_TAB_FIT2 : KX_TAB_FIT1)))
+            times = kTimesFit;
         B.moff = moff;
         B.doff = doff;
         B.ni = (int64_t)a.nx * a.ny * a.nz;
@@ -847,14 +880,14 @@ extern "C" int kx_batch_build(kx_batch *b, const kx_plan *plans, int32_t nprob, 
     const int cus = device_cus();
     const int sp_cu = per_cu(f.spread(c.rb, c.rot, q.dynamic, q.neg_trav), kSpreadBlock,
                              spread_lds(c.rb, nt_max));
-    const int ga_cu = per_cu(f.gather(c.P, c.np, q.dynamic, q.neg_trav), kGatherBlock, 0);
+    const int ga_cu = per_cu(f.gather(c.P, c.np, q.dynamic, times), kGatherBlock, 0);
 
     b->abi_version = KX_ABI_VERSION;
     b->nprob = nprob;
     b->dtype = q.dtype;
     b->tab_fmt = q.tab_fmt;
     b->dynamic = q.dynamic;
-    b->neg_trav = q.neg_trav;
+    b->neg_trav = times;
     b->rblock = c.rb;
     b->sorder = c.rot ? KX_ORDER_ROTATED : KX_ORDER_NATURAL;
     b->gsplit = c.P;

@@ -33,6 +33,13 @@ namespace {
 // same.
 constexpr float kFitBound = 29.5f;  // kWin / 2 less the floor, the pair and a margin
 
+// waves per SIMD asked of the compiler: with two tiles a dynamic group takes
+// 91 vector registers, five waves; six (80 registers, a few words of scratch
+// outside the receiver loop) measured 1.88 -> 1.72 ms on 2D 601x300
+template <typename TD, bool DYN, int NP, int K> struct FitWaves {
+    static constexpr int v = (DYN && NP == 2 && K == 1 && sizeof(TD) == 4) ? 6 : 1;
+};
+
 // lane l + 1's value minus this lane's (lane 63: its own value's negative)
 __device__ __forceinline__ float next_minus(float v)
 {

@@ -37,13 +37,6 @@ int device_cus()
     return cus;
 }
 
-// waves per SIMD asked of the compiler: with two tiles a dynamic group takes
-// 91 vector registers, five waves; six (80 registers, a few words of scratch
-// outside the receiver loop) measured 1.88 -> 1.72 ms on 2D 601x300
-template <typename TD, bool DYN, int NP, int K> struct FitWaves {
-    static constexpr int v = (DYN && NP == 2 && K == 1 && sizeof(TD) == 4) ? 6 : 1;
-};
-
 // the same for plans whose samples all lie in their windows
 template <typename TD, typename TT, bool DYN, int JW, int P, int NP, int K, bool GATE>
 __global__ __launch_bounds__(kGatherBlock, (FitWaves<TD, DYN, NP, K>::v)) void gather_fit_kernel(
