@@ -1562,20 +1562,31 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
 // "same" convolution along time, odd filter
 // ---------------------------------------------------------------------------
 // One workgroup of kConvThreads computes kConvOut consecutive outputs of one
-// trace, kConvPer adjacent outputs per thread.  The flipped filter and the
-// trace window (outputs plus the filter's halo) are staged in LDS, zero
-// padded to whole 4-element groups; a float thread reads both as float4
-// (consecutive lanes read consecutive 16 bytes: no bank conflicts) and keeps
-// the 8 window samples of two groups in registers, so 16 multiply-adds cost
-// two LDS reads.
-
-
-// LDS elements of one convolution workgroup: filter + window + one group of
-// read-ahead
+// trace, kConvPer adjacent outputs per thread.  The trace window (outputs plus
+// the filter's halo) is staged in LDS, zero padded to whole 4-element groups;
+// a float thread reads it as float4 (consecutive lanes read consecutive 16
+// bytes: no bank conflicts) and keeps the 8 window samples of two groups in
+// registers, so 16 multiply-adds cost one LDS read.  The taps are the same in
+// every lane and come through scalar loads, 16 at a time.  The window's loads
+// are in flight together: one after the other, with the taps read from LDS,
+// a launch was bound by their latency (8 x 3751 traces of 1001 samples, 81
+// taps: 167 us, now 93; 24 problems of up to 32 x 256 traces 252 and 149;
+// float64 22 and 14; 21 x 101 traces of 751 samples 15.6 and 10).
+// LDS elements of one convolution workgroup: window + one group of
+// read-ahead, and the filter's length once more (unused; it keeps the longest
+// filter accepted what it was while the taps were staged too)
 __host__ __device__ __forceinline__ int conv_lds_elems(int nh)
 {
     return conv_taps_padded(nh) + kConvOut + conv_taps_padded(nh) + 4;
 }
+
+// adjacent samples in LDS (aligned), and of a row of y (which is not)
+template <typename TD, int N> struct alignas(16) Pack {
+    TD v[N];
+};
+template <typename TD> struct RowPack {
+    TD v[kConvPer];
+};
 
 // Output samples [n0, n0 + kConvOut) of trace tr:
 // y[n] = sum_k h[k] x[n + (nh - 1) / 2 - k], with the trace's signal row
@@ -1587,51 +1598,81 @@ __device__ __forceinline__ void conv_segment(const TD *__restrict__ x, int64_t x
                                              int64_t hstride, int nh, int64_t tr, int n0)
 {
     extern __shared__ __align__(16) unsigned char kx_smem[];
+    typedef const __attribute__((address_space(4))) TD *Taps;
     const int nhp = conv_taps_padded(nh);
-    TD *hs = reinterpret_cast<TD *>(kx_smem);
-    TD *win = hs + nhp;
+    TD *win = reinterpret_cast<TD *>(kx_smem);
     const int c = (nh - 1) / 2;
     const int start = n0 + c - (nh - 1);
     const int nwin = kConvOut + nhp + 4;
     const TD *xr = x + tr * xstride;
-    const TD *hr = h + tr * hstride;
-    for (int k = threadIdx.x; k < nhp; k += blockDim.x)
-        hs[k] = k < nh ? hr[nh - 1 - k] : TD(0);  // flipped: out[i] = sum_k hs[k] win[i + k]
-    for (int j = threadIdx.x; j < nwin; j += blockDim.x) {
+    // the first window samples in flight together, the rest (long filters)
+    // one after the other
+    constexpr int kAhead = kConvPer + 1;
+    TD ahead[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+        ahead[q] = xr[min(max(start + q * kConvThreads + (int)threadIdx.x, 0), nt - 1)];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+        const int j = q * kConvThreads + (int)threadIdx.x, n = start + j;
+        if (j < nwin)
+            win[j] = (n >= 0 && n < nt) ? ahead[q] : TD(0);
+    }
+    for (int j = kAhead * kConvThreads + threadIdx.x; j < nwin; j += kConvThreads) {
         const int n = start + j;
         win[j] = (n >= 0 && n < nt) ? xr[n] : TD(0);
     }
     __syncthreads();
     const int i0 = threadIdx.x * kConvPer;  // first output of this thread
+    // out[i] = sum_k h[nh - 1 - k] win[i + k]
+    const Taps ht = (Taps)(h + tr * hstride) + (nh - 1);
+    const Pack<TD, kConvPer> *w4 = reinterpret_cast<const Pack<TD, kConvPer> *>(win + i0);
     TD acc[kConvPer] = {};
-    if constexpr (sizeof(TD) == 4) {
-        const float4 *w4 = reinterpret_cast<const float4 *>(win) + threadIdx.x;
-        const float4 *h4 = reinterpret_cast<const float4 *>(hs);
-        float4 cur = w4[0];
-        for (int g = 0; g < nhp / 4; ++g) {
-            const float4 nxt = w4[g + 1];
-            const float4 hq = h4[g];
-            const float w[8] = {cur.x, cur.y, cur.z, cur.w, nxt.x, nxt.y, nxt.z, nxt.w};
-            const float hh[4] = {hq.x, hq.y, hq.z, hq.w};
+    Pack<TD, kConvPer> cur = w4[0];
+    auto taps4 = [&](const Pack<TD, kConvPer> &nxt, const TD(&hh)[4]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int r = 0; r < kConvPer; ++r)
-                    acc[r] += hh[q] * w[q + r];
-            cur = nxt;
-        }
-    } else {
-        for (int k = 0; k < nhp; ++k) {
-            const TD hk = hs[k];
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int r = 0; r < kConvPer; ++r)
-                acc[r] += hk * win[i0 + r + k];
-        }
-    }
+                acc[r] = fma(hh[q], q + r < 4 ? cur.v[(q + r) & 3] : nxt.v[(q + r) & 3], acc[r]);
+        cur = nxt;
+    };
+    int k = 0;
+    constexpr int kChunk = 16;
+    for (; k + kChunk <= nh; k += kChunk) {
+        Pack<TD, kConvPer> nx[kChunk / 4];
+        TD hh[kChunk / 4][4];
 #pragma unroll
-    for (int r = 0; r < kConvPer; ++r)
-        if (n0 + i0 + r < nt)
-            y[tr * nt + n0 + i0 + r] = acc[r];
+        for (int g = 0; g < kChunk / 4; ++g) {
+            nx[g] = w4[k / 4 + g + 1];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                hh[g][q] = ht[-(k + 4 * g + q)];
+        }
+#pragma unroll
+        for (int g = 0; g < kChunk / 4; ++g)
+            taps4(nx[g], hh[g]);
+    }
+    for (; k < nhp; k += 4) {
+        TD hh[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            hh[q] = k + q < nh ? ht[-min(k + q, nh - 1)] : TD(0);
+        taps4(w4[k / 4 + 1], hh);
+    }
+    TD *yr = y + tr * nt + n0 + i0;
+    if (n0 + i0 + kConvPer <= nt) {
+        RowPack<TD> out;
+#pragma unroll
+        for (int r = 0; r < kConvPer; ++r)
+            out.v[r] = acc[r];
+        *reinterpret_cast<RowPack<TD> *>(yr) = out;
+    } else {
+#pragma unroll
+        for (int r = 0; r < kConvPer; ++r)
+            if (n0 + i0 + r < nt)
+                yr[r] = acc[r];
+    }
     __syncthreads();  // the window is read before a next item loads its own
 }
 
