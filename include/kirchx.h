@@ -249,7 +249,7 @@ int kx_forward(const kx_plan *p, const void *m, void *d, void *work, void *strea
  * shares the image tiles of a block between several workgroups, each keeping
  * its 64-bit sums in the workspace, and adds them in a second launch (the
  * data are bitwise the same).  kx_forward_work_bytes() is the size with which
- * it runs fastest; kx_forward passes kx_workspace_bytes(p). */
+ * it runs fastest. */
 int64_t kx_forward_work_bytes(const kx_plan *p);
 int kx_forward_ws(const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes,
                   void *stream);

@@ -594,9 +594,28 @@ extern "C" int64_t kx_forward_work_bytes(const kx_plan *p)
     return std::max(b, kx_spread_sums_bytes(p));
 }
 
+// share: bytes of work in which workgroups may share tiles
+static int forward(const kx_plan *p, const void *m, void *d, void *work, int64_t share,
+                   void *stream)
+{
+    if (!p->h || p->nh <= 0)
+        return kx_fail(KX_EINVAL, "forward: wavelet missing");
+    if (!work)
+        return kx_fail(KX_EINVAL, "forward: workspace missing");
+    // one launch where the workgroups can convolve their traces in LDS
+    int rc = kx_spread_wavelet(p, m, d, work, share, stream);
+    if (rc != KX_ENOFUSE)
+        return rc;
+    rc = kx_spread(p, m, work, stream);
+    if (rc)
+        return rc;
+    return kx_conv(work, d, (int64_t)p->ns * p->nr, p->nt, p->h, p->nh, p->dtype, stream);
+}
+
 extern "C" int kx_forward(const kx_plan *p, const void *m, void *d, void *work, void *stream)
 {
-    return kx_forward_ws(p, m, d, work, kx_workspace_bytes(p), stream);
+    int rc = check_plan(p);
+    return rc ? rc : forward(p, m, d, work, 0, stream);
 }
 
 extern "C" int kx_forward_ws(const kx_plan *p, const void *m, void *d, void *work,
@@ -605,21 +624,10 @@ extern "C" int kx_forward_ws(const kx_plan *p, const void *m, void *d, void *wor
     int rc = check_plan(p);
     if (rc)
         return rc;
-    if (!p->h || p->nh <= 0)
-        return kx_fail(KX_EINVAL, "forward: wavelet missing");
-    if (!work)
-        return kx_fail(KX_EINVAL, "forward: workspace missing");
     if (work_bytes < kx_workspace_bytes(p))
         return kx_fail(KX_EINVAL, "forward: workspace of %lld bytes, %lld needed",
                        (long long)work_bytes, (long long)kx_workspace_bytes(p));
-    // one launch where the workgroups can convolve their traces in LDS
-    rc = kx_spread_wavelet(p, m, d, work, work_bytes, stream);
-    if (rc != KX_ENOFUSE)
-        return rc;
-    rc = kx_spread(p, m, work, stream);
-    if (rc)
-        return rc;
-    return kx_conv(work, d, (int64_t)p->ns * p->nr, p->nt, p->h, p->nh, p->dtype, stream);
+    return forward(p, m, d, work, work_bytes, stream);
 }
 
 extern "C" int kx_adjoint(const kx_plan *p, const void *d, void *m, void *work, void *stream)

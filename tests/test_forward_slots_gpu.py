@@ -98,3 +98,21 @@ def test_slot_blocks_shared_tiles(kind):
     with pytest.raises(ValueError, match="workspace"):
         _lib.check(L.kx_forward_ws(ctypes.byref(plan), _lib.ptr(m), _lib.ptr(d), _lib.ptr(work),
                                    base - 1, _lib.stream_ptr(m.device)))
+
+
+def test_forward_leaves_its_workspace_untouched():
+    """kx_forward, whose header says so: no tile is shared through it."""
+    import ctypes
+    import torch
+    from pylops_amd import _lib
+    op, _ = _op(45, 300, nx=131, nz=250, ns=2)
+    m = torch.randn(op.shape[1], generator=torch.Generator().manual_seed(1)).cuda()
+    op.rblock = 16
+    plan, L = op.plan, _lib.load()
+    work = torch.full((L.kx_workspace_bytes(ctypes.byref(plan)),), 7, dtype=torch.uint8,
+                      device=m.device)
+    d = torch.empty(op.shape[0], device=m.device)
+    _lib.check(L.kx_forward(ctypes.byref(plan), _lib.ptr(m), _lib.ptr(d), _lib.ptr(work),
+                            _lib.stream_ptr(m.device)))
+    assert (work == 7).all()
+    assert torch.equal(d, op @ m)
