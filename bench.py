@@ -305,9 +305,10 @@ def build_workload(name, dev):
 
 
 def time_operator(kw, refl, tables, dev, steps, warmup):
-    """A step = kx_forward of the dense image K^T d (the spread with the
-    wavelet convolution in the same launch, plus its two-block scale
-    prepass) + the wavelet correlation of d + kx_gather, i.e. the operator
+    """A step = the forward of the dense image K^T d as the operator runs it
+    (kx_forward_ws: the spread with the wavelet convolution in the same
+    launch, its scale prepass, and where workgroups share tiles the launch
+    that adds their sums) + the wavelet correlation of d + kx_gather, i.e. the operator
     pair of one solver iteration, each part bracketed by HIP events on the
     launch stream.  Returns the timings, the operator and the observed
     data."""
@@ -324,10 +325,11 @@ def time_operator(kw, refl, tables, dev, steps, warmup):
     mt = torch.as_tensor(np.asarray(refl, dtype=np.float32).ravel(), device=dev)
     nd = Op.nsnr * Op.nt
     dobs = torch.empty(nd, dtype=torch.float32, device=dev)
-    work = torch.empty(nd, dtype=torch.float32, device=dev)
+    nwork = max(int(L.kx_forward_work_bytes(pp)), 4 * nd)
+    work = torch.empty(nwork, dtype=torch.uint8, device=dev)
     dcorr = torch.empty(nd, dtype=torch.float32, device=dev)
     img = torch.empty(Op.ni, dtype=torch.float32, device=dev)
-    _lib.check(L.kx_forward(pp, _lib.ptr(mt), _lib.ptr(dobs), _lib.ptr(work), st))
+    _lib.check(L.kx_forward_ws(pp, _lib.ptr(mt), _lib.ptr(dobs), _lib.ptr(work), nwork, st))
     _lib.check(L.kx_adjoint(pp, _lib.ptr(dobs), _lib.ptr(img), _lib.ptr(work), st))
     mdense = img.clone()
     dout = torch.empty_like(dobs)
@@ -336,7 +338,8 @@ def time_operator(kw, refl, tables, dev, steps, warmup):
     def step(ev=None):
         if ev is not None:
             ev[0].record()
-        _lib.check(L.kx_forward(pp, _lib.ptr(mdense), _lib.ptr(dout), _lib.ptr(work), st))
+        _lib.check(L.kx_forward_ws(pp, _lib.ptr(mdense), _lib.ptr(dout), _lib.ptr(work), nwork,
+                                   st))
         if ev is not None:
             ev[1].record()
         _lib.check(L.kx_conv(_lib.ptr(dobs), _lib.ptr(dcorr), Op.nsnr, Op.nt, _lib.ptr(hs),
@@ -365,7 +368,7 @@ def time_operator(kw, refl, tables, dev, steps, warmup):
     res = {"tables": tables, "ms_per_step": round(wall / steps * 1e3, 4),
            "gsamples_s": round(2.0 * trip / (wall / steps) / 1e9, 3),
            "data_gsamples_s": round(2.0 * nd / (wall / steps) / 1e9, 4),
-           # spread: kx_forward (the spread launch with the wavelet
+           # spread: the forward (the spread launch with the wavelet
            # convolution inside it, and its scale prepass)
            "kernel_ms": {"spread": round(t_spread * 1e3, 4),
                          "correlation": round(t_conv * 1e3, 4),
