@@ -43,7 +43,7 @@
 extern "C" {
 #endif
 
-#define KX_ABI_VERSION 5
+#define KX_ABI_VERSION 6
 
 /* Bytes of the per-plan device scratch `aux` (forward accumulation scale). */
 #define KX_AUX_BYTES 4096
@@ -75,6 +75,11 @@ extern "C" {
 #define KX_TAB_FIT1 2
 #define KX_TAB_FIT2 4
 #define KX_TAB_FIT4 8
+/* all of them: a plan with any other bit, or with KX_TAB_SLOTS and KX_F64, is
+ * refused (KX_EINVAL).  What the bits claim cannot be checked: a caller that
+ * fills the tables itself leaves them 0 or sets what kx_slot_table and
+ * kx_table_fit gave. */
+#define KX_TAB_ALL (KX_TAB_SLOTS | KX_TAB_FIT1 | KX_TAB_FIT2 | KX_TAB_FIT4)
 
 /* element types */
 #define KX_F32 0

@@ -370,6 +370,10 @@ int check_plan(const kx_plan *p)
         return kx_fail(KX_ESHAPE, "too many traces");
     if (!p->off_s || !p->base_s || !p->off_r || !p->base_r)
         return kx_fail(KX_EINVAL, "traveltime tables missing");
+    if ((p->tabs & ~KX_TAB_ALL) != 0)
+        return kx_fail(KX_EINVAL, "plan.tabs 0x%x holds unknown bits (KX_TAB_*)", (unsigned)p->tabs);
+    if ((p->tabs & KX_TAB_SLOTS) && p->dtype != KX_F32)
+        return kx_fail(KX_EINVAL, "plan.tabs: slot-ordered tables (KX_TAB_SLOTS) belong to float32 plans");
     if (p->dynamic && (!p->wp_s || !p->wq_s || !p->wp_r || !p->wq_r || !p->izmin))
         return kx_fail(KX_EINVAL, "dynamic weights missing");
     return KX_OK;
