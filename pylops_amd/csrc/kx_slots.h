@@ -51,12 +51,15 @@ template <int N> __device__ __forceinline__ float row_bcast(float v)
 
 // Operations with the value of point N of the lane's run of RB points, v held
 // by the lane of that point.  RB = 8: lanes 0-7 of a row take lane N, lanes
-// 8-15 lane N + 8.  (A DPP instruction must not read a register within two
-// wait states of a vector instruction that wrote it; the compiler sees to it
-// for the builtin, slots_settle for the instructions written here.)
+// 8-15 lane N + 8.  A DPP instruction must not read a register within two
+// wait states of a vector instruction that wrote it.  The compiler sees to it
+// for the builtin but does not look into the instructions written here, and
+// may copy or reload their operands right before them: they wait themselves
+// (2D 601x300 dynamic float32 with 61 x 301 traces 3.49 ms with one wait per
+// tile ahead of all of them, 3.54 so; other shapes 0 to 1% more).
 #define KX_HALF2(OP)                                                                           \
-    OP "_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0x3\n\t" OP                      \
-       "_dpp %0, %1, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xc"
+    "s_nop 1\n\t" OP "_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0x3\n\t" OP       \
+    "_dpp %0, %1, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xc"
 template <int RB, int N> __device__ __forceinline__ float point_add(float v, float x)
 {
     if constexpr (RB == 16)
@@ -317,18 +320,17 @@ __device__ __forceinline__ void slots_body(const KArgs &a, const float *__restri
         cl.txi = more ? cn.txi : cl.txi;
         cl.tyi = more ? cn.tyi : cl.tyi;
         const bool any = c.t < t1 && __ballot(P.mv != 0.f) != 0;
-        float mv = P.mv, os = P.os;
+        float mv = P.mv;
+        const float os = P.os;
         const int base = P.bs + P.br;
         if constexpr (ACC == kAccFix)
             mv = ldexpf(mv, e);
-        int W = ACC == kAccFix && !DYN ? round_half_up(mv) : 0;
+        const int W = ACC == kAccFix && !DYN ? round_half_up(mv) : 0;
         float mps = 0.f, mqs = 0.f;
         if constexpr (DYN) {
             mps = mv * P.ps;
             mqs = mv * P.qs;
         }
-        if constexpr (RB == 8)  // see point_add
-            asm volatile("s_nop 1" : "+v"(os), "+v"(mv), "+v"(W), "+v"(mps), "+v"(mqs));
 #define KX_SLOT(C, I)                                                                          \
     if constexpr (I < CH)                                                                      \
     slot_point<TT, RW, DYN, GATE, NEG, ACC, RB, CH * C + (I < CH ? I : 0)>(                     \

@@ -1,0 +1,29 @@
+"""Properties of the built gfx950 code that the sources rely on and no
+numerical test can show (they hold or fail per build)."""
+import os
+import re
+
+import pytest
+
+from pylops_amd import _lib
+from tests import device_code as D
+
+pytestmark = pytest.mark.skipif(not os.path.exists(os.path.join(D.LLVM, "llvm-objdump")),
+                                reason="the LLVM binary tools are not installed")
+
+
+def test_row_broadcasts_carry_their_wait_states(tmp_path):
+    """A DPP instruction must not read a register within two wait states of
+    the vector instruction that wrote it.  The compiler keeps to it for its
+    own instructions and does not look into inline assembly: every half-row
+    pair written there (bank masks 0x3 and 0xc) follows its own wait."""
+    pairs = 0
+    for name, code in D.disassemble(_lib.LIBPATH, tmp_path, r"slots_kernel.*Li8E"):
+        for i, ins in enumerate(code):
+            if "row_newbcast" not in ins or "bank_mask:0x3" not in ins:
+                continue
+            pairs += 1
+            m = re.match(r"s_nop (\d+)", code[i - 1])
+            assert m and int(m.group(1)) >= 1, (name, code[i - 3:i + 1])
+            assert "row_newbcast" in code[i + 1] and "bank_mask:0xc" in code[i + 1]
+    assert pairs > 100
