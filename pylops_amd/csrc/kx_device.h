@@ -237,13 +237,16 @@ __host__ __device__ __forceinline__ int slot_blocks(int n)
 // ---------------------------------------------------------------------------
 // forward: spread into LDS-resident traces
 // ---------------------------------------------------------------------------
-// LDS accumulation.  For float data every contribution c (rounded to float
-// as the reference rounds it) is added as the integer floor(c * 2^e + 1/2)
-// to a 64-bit fixed-point sample, with one power-of-two scale 2^e per launch
-// chosen from max|m| so that |c| 2^e <= 2^30: the rounding of a contribution
-// is at most 2^-31 of the largest possible one, the sum itself is exact and
+// LDS accumulation.  For float data the weight w of a (point, trace) pair
+// goes to its two samples as integers in a 64-bit fixed point, with one
+// power-of-two scale 2^e per launch chosen from max|m| so that |w| 2^e <
+// 2^30: floor(w f 2^e + 1/2) to the second, and what that leaves of floor(w
+// 2^e + 1/2) to the first (which takes one instruction less than rounding w
+// (1 - f) and keeps the pair's sum).  The first sample's rounding is at most
+// one unit 2^-e, the second's half a unit; the unit is 2^-31 of the bound on
+// the largest contribution (scale_from_stats).  The sum itself is exact and
 // does not depend on the order of the adds, and it cannot overflow (at most
-// 2^32 contributions per sample).  On gfx950 LDS integer atomics sustain
+// 2^31 contributions below 2^31 per sample).  On gfx950 LDS integer atomics sustain
 // ~1.5x the rate of float64 ones and float32 LDS atomics ~1/6 of float64.
 // A launch whose m holds inf or NaN accumulates in float64 instead, so that
 // they propagate as in the reference; double data always does.  So does a
@@ -499,8 +502,7 @@ __device__ __forceinline__ void spread_sample(TC T, int base, TD w, bool on, int
         const TD w1 = w * (TD)f;
         if constexpr (ACC == kAccFix) {
             // fixed point by floor(x + 1/2) in one conversion; the first
-            // sample takes what the second leaves of the rounded weight, so
-            // that the pair's sum is the weight's own rounding
+            // sample takes what the second leaves of the rounded weight
             unsigned long long *acci = static_cast<unsigned long long *>(lds);
             const int i1 = round_half_up(w1);
             const int i0 = round_half_up(w) - i1;
@@ -1089,14 +1091,17 @@ __device__ __forceinline__ void stats_wave(const float *__restrict__ part, int n
 }
 
 // A contribution is at most |m| * wamp * 2 (the truncation path of a
-// negative time weighs a sample by up to 2): e puts that bound below 2^30.
+// negative time weighs a sample by up to 2): e puts that bound, with 2^-16 of
+// it to spare for the float32 products, below 2^31, so that the integers of
+// both samples fit 32 bits.
 // The scaled image values m 2^e are float32: when max|m| 2^e would not be a
 // finite float, or values 2^-40 below the maximum would no longer be normal
 // floats (weights in extreme units), the launch accumulates in float64.
-// A contribution then rounds by at most 2^-30 max|m| wamp, i.e. by
-// 2^-30 R of a typical one, R = max|m| wamp / (mean|m| wtyp) (mean over the
+// A contribution then rounds by at most 2^-29 max|m| wamp (2^-31 of the power
+// of two above 2 max|m| wamp), i.e. by
+// 2^-29 R of a typical one, R = max|m| wamp / (mean|m| wtyp) (mean over the
 // nonzero m; wtyp a typical weight, wamp when not given): when R exceeds
-// kRangeMax = 2^10 (a typical contribution rounding by more than ~2^-20 of
+// kRangeMax = 2^10 (a typical contribution rounding by more than ~2^-19 of
 // itself, and a few 1e-6 of the sums it makes), the launch accumulates in
 // float64 too.
 constexpr double kRangeMax = 1024.0;
@@ -1104,7 +1109,7 @@ constexpr double kRangeMax = 1024.0;
 __device__ __forceinline__ SpreadScale scale_from_stats(float mx, double mean, double wamp,
                                                         double wtyp)
 {
-    const double bound = 2.0 * (double)mx * wamp;
+    const double bound = (2.0 + 0x1p-15) * (double)mx * wamp;
     SpreadScale sc;
     if (!(bound <= 1.7976931348623157e308)) {
         sc.e = 0;
@@ -1115,7 +1120,7 @@ __device__ __forceinline__ SpreadScale scale_from_stats(float mx, double mean, d
     } else {
         int ex;
         frexp(bound, &ex);  // bound < 2^ex
-        sc.e = 30 - ex;
+        sc.e = 31 - ex;
         const double top = ldexp((double)mx, sc.e);
         sc.fixed = (top <= 0x1p126 && ldexp(top, -40) >= 0x1p-126) ? 1 : 0;
         const double wt = wtyp > 0.0 ? wtyp : wamp;
