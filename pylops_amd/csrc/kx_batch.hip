@@ -169,13 +169,15 @@ __global__ __launch_bounds__(kSpreadBlock) void batch_spread_kernel(
 // times of a batch (kx_batch.neg_trav): negative ones; none, and the samples
 // of some problems all in their windows (KX_TAB_FIT*), which take the kernel
 // of kx_fit.h (chosen per item; 24 problems up to 512x256 with float16
-// tables, 21 of which fit: 1.53 -> 1.27 ms); neither
+// tables, 21 of which fit: 1.53 -> 1.27 ms); neither.  The kernel holds both
+// gathers, so its registers are not limited as gather_fit_kernel's are: at six
+// waves per SIMD the general one kept 80 values in scratch memory and a
+// dynamic float32 batch with a problem that does not fit took twice its time
+// (7 problems 450 -> 870 us; now 415; 24 problems 1430 and 1170).
 constexpr int kTimesFit = -1, kTimesAny = 0, kTimesNeg = 1;
 
 template <typename TD, typename TT, bool DYN, int TIMES, int JW, int P, int NP>
-__global__ __launch_bounds__(kGatherBlock,
-                             (TIMES == kTimesFit ? FitWaves<TD, DYN, NP, 1>::v : 1)) void
-batch_gather_kernel(
+__global__ __launch_bounds__(kGatherBlock) void batch_gather_kernel(
     const BatchProb *__restrict__ probs, const GatherItem *__restrict__ items, unsigned *ctr,
     const int *__restrict__ qoff, const TD *__restrict__ d, TD *__restrict__ m)
 {

@@ -27,3 +27,16 @@ def test_row_broadcasts_carry_their_wait_states(tmp_path):
             assert m and int(m.group(1)) >= 1, (name, code[i - 3:i + 1])
             assert "row_newbcast" in code[i + 1] and "bank_mask:0xc" in code[i + 1]
     assert pairs > 100
+
+
+def test_batch_gathers_keep_their_values_in_registers(tmp_path):
+    """The batch adjoint holds the windowed and the general gather in one
+    kernel: with the registers limited for the first, the second kept values
+    of every receiver in scratch memory and took twice its time."""
+    seen = 0
+    for name, md in D.kernel_metadata(_lib.LIBPATH, tmp_path).items():
+        if "batch_gather_kernel" in name:
+            seen += 1
+            assert md["private_segment_fixed_size"] == 0, (name, md)
+            assert md["vgpr_spill_count"] == 0, (name, md)
+    assert seen > 0
