@@ -246,7 +246,8 @@ int kx_xcorr_rows(const void *a, int64_t astride, int32_t la, const void *b, int
  * correlate (convolve with hstar) then gather.  work: kx_workspace_bytes.
  * A float32 forward whose workgroups hold their traces as 64-bit sums
  * convolves them in LDS in the same launch (the data are bitwise those of
- * kx_spread followed by kx_conv) and leaves work untouched. */
+ * kx_spread followed by kx_conv) and leaves work untouched, except where its
+ * filter is so long that the two launches are faster. */
 int kx_forward(const kx_plan *p, const void *m, void *d, void *work, void *stream);
 
 /* kx_forward with a workspace of work_bytes >= kx_workspace_bytes(p): a

@@ -606,8 +606,8 @@ static int forward(const kx_plan *p, const void *m, void *d, void *work, int64_t
         return kx_fail(KX_EINVAL, "forward: wavelet missing");
     if (!work)
         return kx_fail(KX_EINVAL, "forward: workspace missing");
-    // one launch where the workgroups can convolve their traces in LDS
-    int rc = kx_spread_wavelet(p, m, d, work, share, stream);
+    // one launch where the workgroups convolve their traces in LDS
+    int rc = kx_spread_wavelet(p, m, d, work, share, true, stream);
     if (rc != KX_ENOFUSE)
         return rc;
     rc = kx_spread(p, m, work, stream);

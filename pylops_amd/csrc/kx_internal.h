@@ -16,11 +16,13 @@ extern "C" __attribute__((visibility("hidden"))) int kx_plan_check(const kx_plan
 #define KX_ENOFUSE (-100)
 
 // The forward operator in one launch: the spread of m convolved with the
-// plan's wavelet into d, or KX_ENOFUSE.  With work_bytes of scratch at work
+// plan's wavelet into d, or KX_ENOFUSE (with two_launches also where the
+// spread and the convolution are faster apart).  With work_bytes of scratch at work
 // the tiles of a receiver block may be shared by several workgroups, a second
 // launch adding their sums.
 extern "C" __attribute__((visibility("hidden"))) int kx_spread_wavelet(
-    const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes, void *stream);
+    const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes, bool two_launches,
+    void *stream);
 // The scratch with which kx_spread_wavelet runs in its fastest shape.
 extern "C" __attribute__((visibility("hidden"))) int64_t kx_spread_sums_bytes(const kx_plan *p);
 

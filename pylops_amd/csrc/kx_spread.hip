@@ -271,64 +271,188 @@ int launch_spread_o(KArgs a, int requested, int max_rb, const void *m, void *y,
     }
 }
 
+// Whether the kernels of 4, 2 and 1 block sources (see launch_spread_d;
+// float16 plans keep the two sides' offsets in different types and block
+// receivers).
+bool blocks_sources(const kx_plan *p)
+{
+    if (p->dtype != KX_F32 || p->tab_fmt == KX_F16)
+        return false;
+    return p->sside == KX_SIDE_AUTO ? p->ny == 1 && p->ns < p->nr : p->sside == KX_SIDE_SOURCES;
+}
+
 // How a forward runs in slot blocks: rb receivers per workgroup (0: the
 // kernels of 4, 2 and 1), the pairs past the first nfull in `parts`
-// workgroups each.
+// workgroups each; fused: the wavelet convolved in the same launch.
 struct SlotsShape {
     int rb, threads, nfull, parts;
+    bool fused;
     size_t lds, sums_bytes;
 };
 
-// The shape with the smallest estimated time, in clocks of a CU.  A CU's
-// clocks per tile and receiver, with all its waves, were measured at: blocks
-// of 4, 2 or 1 27 kinematic and 36 dynamic; slots of 16 17 (float32 tables,
-// 3D 128x128x120 with 25 x 400) and 15 (float16), dynamic 30 (2D 201x121
-// with 21 x 101; float16 333x187 with 37 x 149); slots of 8 a quarter more,
-// dynamic 32 (601x300 with 61 x 301).  A workgroup spends about 18000
-// clocks on its scale, first loads, clearing and writing out.  Where the
-// pairs are no multiple of the workgroups that run at once, the last ones are
-// shared by several workgroups, which costs their sums' way through memory
-// (about 1000 bytes per clock).  The estimates miss by up to 8%: the slots have
-// to gain as much.  A requested block size is an upper bound.
-SlotsShape pick_slots(const kx_plan *p, int nh, int64_t work_bytes)
+// Estimated times of a forward, in microseconds: sums of terms whose factors
+// were fitted to the measured times of 579 random 2D and 3D operators (64 to
+// 5000 tiles, 1 to 61 sources, 2 to 400 receivers, 200 to 2500 samples, 41 to
+// 2400 taps; 9300 launches, 90% of them within 12%).
+//   fixed   the launches
+//   round   a round of workgroups
+//   clear   clearing and writing out, per 1000 samples of a CU
+//   step    a wave's (tile, receiver), the instructions and LDS operations of
+//           all waves of a CU, per 1000
+//   chain   the same where one wave's own chain of operations is as long
+//   tile    a wave's tile (its loads' latency), per 1000
+//   conv    per 10^6 multiply-adds of a CU
+struct RowsTime {
+    double fixed, clear, step, chain, conv, tile;
+};
+struct SlotsTime {
+    double fixed, round, clear, step, chain, conv;
+    double add;       // adding the parts: per 100 dependent loads of a thread
+    double bytes;     // ... per MB of sums
+    double add_conv;  // ... its convolution, per 1000 four-tap steps of a thread
+};
+constexpr RowsTime kRowsTime[2] = {  // kinematic, dynamic
+    {7.35, 0.63, 7.97, 12.3, 10.5, 248.0},
+    {8.87, 0.57, 10.3, 2.3, 11.7, 280.0},
+};
+constexpr SlotsTime kSlotsTime[2][2][2] = {  // [dynamic][blocks of 16][1024 threads]
+    {{{10.8, 0, 0, 4.73, 71.1, 12.7, 36.9, 0.342, 75.4},
+      {11.8, 2.14, 0, 11.7, 0, 10.3, 38.3, 0.309, 55.3}},
+     {{10.4, 0, 0.0234, 4.13, 43.7, 9.91, 35.7, 0.52, 78.2},
+      {5, 7.68, 0.066, 7.89, 0, 9.49, 35, 0.309, 73.5}}},
+    {{{10.9, 0.757, 0.0304, 7.87, 47.6, 14.6, 35.3, 0.344, 71.8},
+      {8.18, 3.28, 0.251, 11.3, 0, 16.1, 36.5, 0.172, 67.7}},
+     {{10.6, 0, 0.125, 6.42, 37.2, 12.4, 33.7, 0.479, 76.8},
+      {3.06, 6.75, 0.256, 9.03, 0, 10.1, 34.9, 0.329, 69.8}}},
+};
+
+// one(w) summed over the rounds of wgs workgroups, `at_once` at a time
+template <typename F> double sum_rounds(int64_t wgs, int64_t at_once, F one)
 {
-    SlotsShape best{0, 0, 0, 1, 0, 0};
-    if (!(p->tabs & KX_TAB_SLOTS) || p->dtype != KX_F32 || p->sside == KX_SIDE_SOURCES)
+    double t = (double)(wgs / at_once) * (wgs >= at_once ? one(at_once) : 0.0);
+    return wgs % at_once ? t + one(wgs % at_once) : t;
+}
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// kx_conv of the traces
+double conv_time(const kx_plan *p, int nh, int cus)
+{
+    const double ntr = (double)p->ns * p->nr;
+    return 7.2 + 19.3e-9 * ntr * p->nt * nh +
+           6.5e-3 * nh * std::ceil(ntr * ceil_div(p->nt, kConvOut) / (4.0 * cus));
+}
+
+// the kernels of 4, 2 and 1, in the block that pick_rblock takes (with its
+// registers' share of the occupancy as measured)
+double rows_time(const kx_plan *p, int nh, int cus)
+{
+    const RowsTime &M = kRowsTime[p->dynamic != 0];
+    const bool xs = blocks_sources(p);
+    const int64_t n = xs ? p->ns : p->nr, other = xs ? p->nr : p->ns;
+    int rb = 1, per_cu = 1;
+    double best = -1.0;
+    for (int c : kRblocks) {
+        if (spread_lds_bytes(c, p->nt) > lds_budget() || (c > 1 && c / 2 >= n))
+            continue;
+        const int k = std::min((int)(kLdsPerCu / spread_lds_bytes(c, p->nt)), p->dynamic ? 3 : 4);
+        const double score = std::min(24.0, (double)k * kSpreadWaves) / 24.0 * k * std::min<int64_t>(c, n);
+        if (score > best * 1.0001) {
+            best = score;
+            rb = c;
+            per_cu = k;
+        }
+    }
+    const bool fused = nh > 0 && fused_conv_ok(rb, p->nt, nh, spread_lds_bytes(rb, p->nt),
+                                               kSpreadBlock);
+    const double tiles = (double)ceil_div(p->ntiles, kSpreadWaves);
+    const double t = sum_rounds(other * ceil_div(n, rb), (int64_t)cus * per_cu, [&](int64_t w) {
+        const double k = (double)ceil_div(w, cus);
+        return 1e-3 * (k * p->nt * rb * M.clear + tiles * (M.tile + rb * (M.chain + kSpreadWaves * k * M.step))) +
+               (fused ? 1e-6 * k * rb * p->nt * nh * M.conv : 0.0);
+    });
+    return M.fixed + t + (nh > 0 && !fused ? conv_time(p, nh, cus) : 0.0);
+}
+
+// a slot shape, convolving with nh taps (0: none)
+double slots_time(const kx_plan *p, const SlotsShape &g, int nh, int cus)
+{
+    const SlotsTime &M =
+        kSlotsTime[p->dynamic != 0][g.rb == 16][g.threads == kSlotsMaxThreads];
+    const int nw = g.threads / kWave;
+    const int64_t at_once = (int64_t)cus * (kSlotsMaxThreads / g.threads);
+    const int64_t nrest = p->ns * ceil_div(p->nr, g.rb) - g.nfull;
+    auto rounds = [&](int64_t wgs, int64_t tiles, int taps) {
+        const double steps = (double)ceil_div(tiles, nw);
+        return sum_rounds(wgs, at_once, [&](int64_t w) {
+            const double k = (double)ceil_div(w, cus);
+            return M.round + 1e-3 * g.rb * (k * p->nt * M.clear + steps * (M.chain + nw * k * M.step)) +
+                   1e-6 * k * g.rb * p->nt * taps * M.conv;
+        });
+    };
+    double t = M.fixed + rounds(g.nfull, p->ntiles, nh);
+    if (g.parts > 1) {
+        const double wgs = (double)nrest * (g.rb / kFinalRows);
+        const double loads = (double)ceil_div((int64_t)p->nt * kFinalRows, kBlock) *
+                             (g.parts / 4 + g.parts % 4);
+        t += rounds(nrest * g.parts, ceil_div(p->ntiles, g.parts), 0) +
+             1e-2 * M.add * loads * std::max(1.0, wgs / (4.0 * cus)) +
+             1e-6 * M.bytes * (double)g.sums_bytes +
+             1e-3 * M.add_conv * (double)ceil_div(p->nt, kBlock) * (conv_taps_padded(nh) / 4) *
+                 std::max(1.0, wgs / (2.0 * cus));
+    }
+    return t;
+}
+
+// The shape with the smallest estimated time; the slots have to be 2% faster
+// than the kernels of 4, 2 and 1.  Where the pairs are no multiple of the
+// workgroups that run at once, the last ones may be shared by several
+// workgroups, in work_bytes of scratch, whose sums a second launch adds (four
+// loads of a thread in flight: counts of parts that are no multiple of 4
+// wait longer).  Long filters are convolved by a launch of their own
+// (unfused, where the caller can: two_launches), with the whole chip instead
+// of the workgroups that hold the traces: 201x150 with 21 x 101 traces of
+// 1201 samples, 1139 taps, 414 us in LDS and 214 so.  A requested block size
+// is an upper bound, without a comparison with smaller ones than 8.
+SlotsShape pick_slots(const kx_plan *p, int nh, int64_t work_bytes, bool two_launches)
+{
+    SlotsShape best{0, 0, 0, 1, false, 0, 0};
+    if (!(p->tabs & KX_TAB_SLOTS) || p->dtype != KX_F32 || p->sside == KX_SIDE_SOURCES ||
+        (p->rblock > 0 && p->rblock < 8))
         return best;
     const int cus = device_cus();
-    const bool half = p->tab_fmt == KX_F16;
-    const double fixed = 18000.0, tiles = (double)p->ntiles;
-    double best_t = 1e300;
-    if (p->rblock == 0) {  // what the kernels of 4 would take
-        const double pairs = (double)p->ns * ((p->nr + 3) / 4);
-        best_t = 0.92 * (std::ceil(pairs / cus) * tiles * 4 * (p->dynamic ? 36.0 : 27.0) + fixed);
-    }
+    double best_t = p->rblock == 0 ? 0.98 * rows_time(p, nh, cus) : 1e300;
+    auto consider = [&](SlotsShape g) {
+        const double t = nh > 0 && !g.fused
+                             ? 1.05 * (slots_time(p, g, 0, cus) + conv_time(p, nh, cus))
+                             : slots_time(p, g, nh, cus);
+        if (t < best_t * 0.99) {
+            best_t = t;
+            best = g;
+        }
+    };
     for (int rb : {16, 8}) {
         if (p->rblock > 0 && rb > p->rblock)
             continue;
+        const int64_t pairs = p->ns * ceil_div(p->nr, rb);
+        if (nh > 0 && two_launches)
+            if (const int th = slots_threads(rb, p->nt, 0))
+                consider({rb, th, (int)pairs, 1, false, slots_lds_bytes(rb, p->nt, 0), 0});
         const int th = slots_threads(rb, p->nt, nh);
         if (!th)
             continue;
-        const int per_cu = kSlotsMaxThreads / th, at_once = cus * per_cu;
-        const int64_t pairs = (int64_t)p->ns * ((p->nr + rb - 1) / rb);
-        const double step = p->dynamic ? (rb == 8 ? 32.0 : 30.0)
-                                       : (half ? 15.0 : 17.0) * (rb == 8 ? 1.25 : 1.0);
-        const double work = tiles * rb * step * per_cu, c0 = fixed + p->nt * rb / th * 60.0;
-        for (int parts = 1; parts <= 16; ++parts) {
-            const int64_t nfull = parts > 1 ? pairs / at_once * at_once : pairs;
-            const int64_t nrest = pairs - nfull;
-            const size_t sums = parts > 1 ? (size_t)(nrest * parts) * p->nt * rb * 8 : 0;
-            if (parts > 1 && (nh <= 0 || nrest == 0 || (int64_t)sums > work_bytes ||
-                              p->ntiles < (int64_t)parts * (th / kWave)))
+        const size_t lds = slots_lds_bytes(rb, p->nt, nh);
+        consider({rb, th, (int)pairs, 1, nh > 0, lds, 0});
+        if (nh <= 0)
+            continue;
+        const int64_t at_once = (int64_t)cus * (kSlotsMaxThreads / th);
+        const int64_t nfull = pairs / at_once * at_once, nrest = pairs - nfull;
+        for (int parts : {2, 3, 4, 5, 6, 8, 10, 12, 14, 16}) {
+            const size_t sums = (size_t)(nrest * parts) * p->nt * rb * 8;
+            if (nrest == 0 || (int64_t)sums > work_bytes ||
+                p->ntiles < (int64_t)parts * (th / kWave))
                 break;
-            double t = std::ceil((double)nfull / at_once) * (work + c0);
-            if (parts > 1)
-                t += std::ceil((double)nrest * parts / at_once) * (work / parts + c0) + 15000.0 +
-                     2.0 * sums / 1000.0;
-            if (t < best_t * 0.98) {
-                best_t = t;
-                best = {rb, th, (int)nfull, parts, slots_lds_bytes(rb, p->nt, nh), sums};
-            }
+            consider({rb, th, (int)nfull, parts, true, lds, sums});
         }
     }
     return best;
@@ -426,10 +550,12 @@ int launch_spread_seg(const KArgs &a, const void *m, void *y, const SpreadScale 
     return KX_OK;
 }
 
-// work: work_bytes of scratch for the parts of slot blocks (0: one part).
+// work: work_bytes of scratch for the parts of slot blocks (0: one part);
+// two_launches: whether the caller convolves by itself after KX_ENOFUSE.
 template <typename TD, typename TT>
 int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream_t st,
-                    const void *h = nullptr, void *work = nullptr, int64_t work_bytes = 0)
+                    const void *h = nullptr, void *work = nullptr, int64_t work_bytes = 0,
+                    bool two_launches = false)
 {
     const int nh = h != nullptr ? p->nh : 0;
     if (h != nullptr && sizeof(TD) != 4)
@@ -444,13 +570,10 @@ int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream
     // registers per lane grow with the block: keep two workgroups per CU
     const int max_rb = 4;
     SpreadScale *sc = reinterpret_cast<SpreadScale *>(p->aux);
-    const SlotsShape slots = pick_slots(p, nh, work ? work_bytes : 0);
-    int side = p->sside;
-    if (side == KX_SIDE_AUTO)
-        side = (p->ny == 1 && p->ns < p->nr) ? KX_SIDE_SOURCES : KX_SIDE_RECEIVERS;
-    // (float16 plans keep the two sides' offsets in different types and
-    // block receivers)
-    const bool xs = sizeof(TD) == 4 && side == KX_SIDE_SOURCES && p->tab_fmt != KX_F16;
+    const SlotsShape slots = pick_slots(p, nh, work ? work_bytes : 0, two_launches);
+    if (slots.rb && h != nullptr && !slots.fused)
+        return KX_ENOFUSE;
+    const bool xs = blocks_sources(p);
     if constexpr (sizeof(TD) == 4) {
         // fixed-point scale of this launch from max|m|
         const int64_t ni = (int64_t)p->nx * p->ny * p->nz;
@@ -531,7 +654,8 @@ extern "C" int kx_spread(const kx_plan *p, const void *m, void *traces, void *st
 }
 
 extern "C" __attribute__((visibility("hidden"))) int kx_spread_wavelet(
-    const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes, void *stream)
+    const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes, bool two_launches,
+    void *stream)
 {
     int rc = kx_plan_check(p);
     if (rc)
@@ -543,13 +667,13 @@ extern "C" __attribute__((visibility("hidden"))) int kx_spread_wavelet(
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const KArgs a = make_args(p);
     if (p->tab_fmt == KX_F16)
-        return launch_spread_d<float, __half>(p, a, m, d, st, p->h, work, work_bytes);
-    return launch_spread_d<float, float>(p, a, m, d, st, p->h, work, work_bytes);
+        return launch_spread_d<float, __half>(p, a, m, d, st, p->h, work, work_bytes, two_launches);
+    return launch_spread_d<float, float>(p, a, m, d, st, p->h, work, work_bytes, two_launches);
 }
 
 extern "C" __attribute__((visibility("hidden"))) int64_t kx_spread_sums_bytes(const kx_plan *p)
 {
-    return (int64_t)pick_slots(p, p->nh, INT64_MAX).sums_bytes;
+    return (int64_t)pick_slots(p, p->nh, INT64_MAX, true).sums_bytes;
 }
 
 namespace {
@@ -706,7 +830,13 @@ extern "C" int kx_forward_noalloc(const kx_plan *p, const void *m, void *d, void
     // clearing)
     kx_plan q = *p;
     q.aux = s;
-    rc = kx_spread_wavelet(&q, m, d, nullptr, 0, stream);
+    rc = kx_spread_wavelet(&q, m, d, nullptr, 0, false, stream);
+    if (rc == KX_ENOFUSE && q.rblock == 0 && (q.tabs & KX_TAB_SLOTS)) {
+        // filters too long for the rows of the estimated fastest shape may
+        // fit a slot block, whose LDS is not bound to the sums' size
+        q.rblock = 16;
+        rc = kx_spread_wavelet(&q, m, d, nullptr, 0, false, stream);
+    }
     if (rc == KX_ENOFUSE)
         return kx_failf(KX_ELDS,
                         "forward_noalloc: this plan's forward cannot convolve in the spread "
