@@ -66,13 +66,26 @@ int launch_gather_p(KArgs a, const void *d, int64_t dstride, void *m, int64_t ms
     if constexpr (!NEG) {
         // Plans with a sample outside the windows, or whose block of sources
         // is too large for 31-bit byte offsets, and negative times take the
-        // general kernel.  So do launches of less than a wave per SIMD, which
-        // wait for memory, not for instructions: the adjoint of a 101x100
-        // grid, 11 x 51 traces, 27.5 us there and 28.6 here (a dynamic
-        // 121x81 gather 37.8 and 38.8); 201x101, 20 x 51 traces, the gather
-        // alone 37.9 and 31.8, 301x201 dynamic 117 and 90.
+        // general kernel.  So do launches that wait for memory more than for
+        // instructions, which the general kernel has fewer of in flight
+        // between its loads and their use (both measured on 1970 random
+        // gathers of 1 to 16 sources; the times are general and windowless):
+        //  - less than a wave per SIMD (121x81 dynamic 37.8 and 38.8 us);
+        //  - one or two tiles per wave, and no more sources than half the
+        //    wave's slots (581x394, 2 x 240 traces, 92 and 111 us; 592 such
+        //    gathers 1% slower in the middle and up to 25%; with four tiles
+        //    the windowless kernel is a quarter faster there too);
+        //  - kinematic float32, less than two waves per SIMD and one pass
+        //    over the sources (313x368, 3 x 117 traces, 49 and 58 us; with
+        //    more passes 0 to 25% faster, as dynamic and float64 gathers
+        //    are).
+        // Several models per wave share the windows' addresses (26 launches
+        // of 1 or 2 sources: 0.91 to 1.06 times, 0.98 in the middle).
         constexpr int fit = NP == 4 ? KX_TAB_FIT4 : (NP == 2 ? KX_TAB_FIT2 : KX_TAB_FIT1);
-        if ((a.tabs & fit) && nblk >= device_cus() &&
+        const int cus = device_cus();
+        const bool slots_used = NP == 4 || K > 1 || a.ns > JW * P / 2;
+        const bool hidden = K > 1 || DYN || sizeof(TD) == 8 || nblk >= 2 * cus || a.ns > JW * P;
+        if ((a.tabs & fit) && nblk >= cus && slots_used && hidden &&
             (int64_t)JW * P * a.nr * a.nt * (int64_t)sizeof(TD) < ((int64_t)1 << 30)) {
             hipLaunchKernelGGL((gather_fit_kernel<TD, TT, DYN, JW, P, NP, K, GATE>), dim3(nblk),
                                dim3(kGatherBlock), 0, st, a, reinterpret_cast<const TD *>(d),
