@@ -94,13 +94,13 @@ extern "C" const char *kx_last_error(void) { return g_err; }
 // ---------------------------------------------------------------------------
 namespace {
 
-template <typename TD>
+template <typename TD, bool LONG>
 __global__ __launch_bounds__(kConvThreads) void conv_kernel(const TD *__restrict__ x, int64_t xstride,
                                                       TD *__restrict__ y, int nt,
                                                       const TD *__restrict__ h, int64_t hstride,
                                                       int nh, int nseg)
 {
-    conv_segment<TD>(x, xstride, y, nt, h, hstride, nh, blockIdx.x / nseg,
+    conv_segment<TD, LONG>(x, xstride, y, nt, h, hstride, nh, blockIdx.x / nseg,
                      (blockIdx.x % nseg) * kConvOut);
 }
 
@@ -541,12 +541,16 @@ extern "C" int kx_conv_rows(const void *x, int64_t xstride, void *y, int64_t ntr
         return kx_fail(KX_ELDS, "conv: filter of %d taps does not fit LDS", nh);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const dim3 grid((unsigned)(ntr * nseg));
-    if (dtype == KX_F32)
-        hipLaunchKernelGGL(conv_kernel<float>, grid, dim3(kConvThreads), lds, st,
+    if (dtype == KX_F32 && nh >= kLongFilter)
+        hipLaunchKernelGGL((conv_kernel<float, true>), grid, dim3(kConvThreads), lds, st,
+                           reinterpret_cast<const float *>(x), xstride, reinterpret_cast<float *>(y),
+                           nt, reinterpret_cast<const float *>(h), hstride, nh, nseg);
+    else if (dtype == KX_F32)
+        hipLaunchKernelGGL((conv_kernel<float, false>), grid, dim3(kConvThreads), lds, st,
                            reinterpret_cast<const float *>(x), xstride, reinterpret_cast<float *>(y),
                            nt, reinterpret_cast<const float *>(h), hstride, nh, nseg);
     else if (dtype == KX_F64)
-        hipLaunchKernelGGL(conv_kernel<double>, grid, dim3(kConvThreads), lds, st,
+        hipLaunchKernelGGL((conv_kernel<double, false>), grid, dim3(kConvThreads), lds, st,
                            reinterpret_cast<const double *>(x), xstride,
                            reinterpret_cast<double *>(y), nt, reinterpret_cast<const double *>(h),
                            hstride, nh, nseg);

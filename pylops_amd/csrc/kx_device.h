@@ -1577,9 +1577,15 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
 // a launch was bound by their latency (8 x 3751 traces of 1001 samples, 81
 // taps: 167 us, now 93; 24 problems of up to 32 x 256 traces 252 and 149;
 // float64 22 and 14; 21 x 101 traces of 751 samples 15.6 and 10).
+// A filter of fewer than 16 taps has no chunk, only groups of four, each of
+// which would wait for its scalar loads: its taps are staged in LDS with the
+// window (20000 traces of 128 samples, 15 taps: 13.0 us, 20.0 with scalar
+// loads).  Long filters of float32 data take 32 taps at a time (LONG, a kernel
+// of its own: with both loops in one the compiler made the shorter 1.6 times
+// slower): 300 traces of 64 samples, 1001 taps, 21.1 and 19.1 us.
 // LDS elements of one convolution workgroup: window + one group of
-// read-ahead, and the filter's length once more (unused; it keeps the longest
-// filter accepted what it was while the taps were staged too)
+// read-ahead, and the filter's length once more (the taps of a short filter;
+// it also keeps the longest filter accepted what it was while all were staged)
 __host__ __device__ __forceinline__ int conv_lds_elems(int nh)
 {
     return conv_taps_padded(nh) + kConvOut + conv_taps_padded(nh) + 4;
@@ -1593,11 +1599,14 @@ template <typename TD> struct RowPack {
     TD v[kConvPer];
 };
 
+// taps from which a float32 convolution takes 32 at a time
+constexpr int kLongFilter = 256;
+
 // Output samples [n0, n0 + kConvOut) of trace tr:
 // y[n] = sum_k h[k] x[n + (nh - 1) / 2 - k], with the trace's signal row
 // at x + tr * xstride and its filter at h + tr * hstride (a stride of 0
 // shares one row between all traces); y rows are nt apart.
-template <typename TD>
+template <typename TD, bool LONG = false>
 __device__ __forceinline__ void conv_segment(const TD *__restrict__ x, int64_t xstride,
                                              TD *__restrict__ y, int nt, const TD *__restrict__ h,
                                              int64_t hstride, int nh, int64_t tr, int n0)
@@ -1617,6 +1626,10 @@ __device__ __forceinline__ void conv_segment(const TD *__restrict__ x, int64_t x
 #pragma unroll
     for (int q = 0; q < kAhead; ++q)
         ahead[q] = xr[min(max(start + q * kConvThreads + (int)threadIdx.x, 0), nt - 1)];
+    TD *hs = win + nwin;  // the taps of a filter without a chunk, flipped
+    constexpr int kChunk = 16;
+    if (!LONG && nh < kChunk && (int)threadIdx.x < nhp)
+        hs[threadIdx.x] = (int)threadIdx.x < nh ? h[tr * hstride + nh - 1 - threadIdx.x] : TD(0);
 #pragma unroll
     for (int q = 0; q < kAhead; ++q) {
         const int j = q * kConvThreads + (int)threadIdx.x, n = start + j;
@@ -1643,20 +1656,36 @@ __device__ __forceinline__ void conv_segment(const TD *__restrict__ x, int64_t x
         cur = nxt;
     };
     int k = 0;
-    constexpr int kChunk = 16;
-    for (; k + kChunk <= nh; k += kChunk) {
-        Pack<TD, kConvPer> nx[kChunk / 4];
-        TD hh[kChunk / 4][4];
+    // N taps: their scalar loads and window reads wait once
+    auto chunk = [&](auto len) __attribute__((always_inline)) {
+        constexpr int N = decltype(len)::value;
+        Pack<TD, kConvPer> nx[N / 4];
+        TD hh[N / 4][4];
 #pragma unroll
-        for (int g = 0; g < kChunk / 4; ++g) {
+        for (int g = 0; g < N / 4; ++g) {
             nx[g] = w4[k / 4 + g + 1];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 hh[g][q] = ht[-(k + 4 * g + q)];
         }
 #pragma unroll
-        for (int g = 0; g < kChunk / 4; ++g)
+        for (int g = 0; g < N / 4; ++g)
             taps4(nx[g], hh[g]);
+        k += N;
+    };
+    if constexpr (LONG) {
+        while (k + 2 * kChunk <= nh)
+            chunk(IntC<2 * kChunk>{});
+        if (k + kChunk <= nh)
+            chunk(IntC<kChunk>{});
+    } else {
+        while (k + kChunk <= nh)
+            chunk(IntC<kChunk>{});
+    }
+    if (!LONG && nh < kChunk) {
+        const Pack<TD, 4> *h4 = reinterpret_cast<const Pack<TD, 4> *>(hs);
+        for (; k < nhp; k += 4)
+            taps4(w4[k / 4 + 1], h4[k / 4].v);
     }
     for (; k < nhp; k += 4) {
         TD hh[4];
