@@ -344,8 +344,9 @@ double conv_time(const kx_plan *p, int nh, int cus)
 }
 
 // the kernels of 4, 2 and 1, in the block that pick_rblock takes (with its
-// registers' share of the occupancy as measured)
-double rows_time(const kx_plan *p, int nh, int cus)
+// registers' share of the occupancy as measured); a caller without a second
+// launch (kx_forward_noalloc) compares shapes that convolve in their own
+double rows_time(const kx_plan *p, int nh, int cus, bool two_launches)
 {
     const RowsTime &M = kRowsTime[p->dynamic != 0];
     const bool xs = blocks_sources(p);
@@ -363,8 +364,9 @@ double rows_time(const kx_plan *p, int nh, int cus)
             per_cu = k;
         }
     }
-    const bool fused = nh > 0 && fused_conv_ok(rb, p->nt, nh, spread_lds_bytes(rb, p->nt),
-                                               kSpreadBlock);
+    const bool fused =
+        nh > 0 && (!two_launches || fused_conv_ok(rb, p->nt, nh, spread_lds_bytes(rb, p->nt),
+                                                  kSpreadBlock));
     const double tiles = (double)ceil_div(p->ntiles, kSpreadWaves);
     const double t = sum_rounds(other * ceil_div(n, rb), (int64_t)cus * per_cu, [&](int64_t w) {
         const double k = (double)ceil_div(w, cus);
@@ -421,7 +423,7 @@ SlotsShape pick_slots(const kx_plan *p, int nh, int64_t work_bytes, bool two_lau
         (p->rblock > 0 && p->rblock < 8))
         return best;
     const int cus = device_cus();
-    double best_t = p->rblock == 0 ? 0.98 * rows_time(p, nh, cus) : 1e300;
+    double best_t = p->rblock == 0 ? 0.98 * rows_time(p, nh, cus, two_launches) : 1e300;
     auto consider = [&](SlotsShape g) {
         const double t = nh > 0 && !g.fused
                              ? 1.05 * (slots_time(p, g, 0, cus) + conv_time(p, nh, cus))
@@ -831,9 +833,10 @@ extern "C" int kx_forward_noalloc(const kx_plan *p, const void *m, void *d, void
     kx_plan q = *p;
     q.aux = s;
     rc = kx_spread_wavelet(&q, m, d, nullptr, 0, false, stream);
-    if (rc == KX_ENOFUSE && q.rblock == 0 && (q.tabs & KX_TAB_SLOTS)) {
+    if (rc == KX_ENOFUSE && q.rblock == 0 && (q.tabs & KX_TAB_SLOTS) && q.nr > 4) {
         // filters too long for the rows of the estimated fastest shape may
-        // fit a slot block, whose LDS is not bound to the sums' size
+        // fit a slot block, whose LDS is not bound to the sums' size (plans
+        // that would leave half of it empty stay refused)
         q.rblock = 16;
         rc = kx_spread_wavelet(&q, m, d, nullptr, 0, false, stream);
     }
