@@ -186,6 +186,11 @@ int kx_tile_table(const kx_plan *geom, const double *tabT, int32_t n,
  * table (KX_TAB_SLOTS): per tile and block of 16 receivers, chunks of 16
  * bytes of consecutive points of one receiver, so that the lanes of a wave
  * read contiguous memory.  (No reference counterpart: device layout.) */
+/* kx_forward_slots: 1 if a forward (kx_forward, kx_forward_ws or kx_spread) of
+ * this plan would read the copies, 0 if they would only take memory; it looks
+ * at the geometry, ns, nr, nt, nh, dtype, tab_fmt, dynamic, rblock and sside
+ * alone (no table needs to exist). */
+int kx_forward_slots(const kx_plan *p);
 int64_t kx_slot_table_elems(const kx_plan *geom, int32_t n);
 int kx_slot_table(const kx_plan *geom, int32_t n, int32_t fmt, void *tab, void *stream);
 

@@ -23,7 +23,7 @@ KX_EINVAL, KX_ESHAPE, KX_ETYPE, KX_EABI, KX_ELDS = -1, -2, -3, -4, -5
 
 EXPORTS = (
     "kx_version", "kx_last_error", "kx_workspace_bytes", "kx_encode_table",
-    "kx_tile_table", "kx_slot_table_elems", "kx_slot_table", "kx_table_fit", "kx_spread",
+    "kx_tile_table", "kx_forward_slots", "kx_slot_table_elems", "kx_slot_table", "kx_table_fit", "kx_spread",
     "kx_gather", "kx_conv", "kx_forward", "kx_forward_work_bytes", "kx_forward_ws",
     "kx_adjoint", "kx_reduce_workspace_bytes", "kx_dot",
     "kx_solver_workspace_bytes", "kx_vec", "kx_dot_dev", "kx_lsqr_xw",
@@ -192,6 +192,7 @@ def _declare(L):
         "kx_workspace_bytes": ([PP], I64),
         "kx_encode_table": ([PP, P, I32, D, I32, P, P, P], ctypes.c_int),
         "kx_tile_table": ([PP, P, I32, I32, P, P], ctypes.c_int),
+        "kx_forward_slots": ([PP], ctypes.c_int),
         "kx_slot_table_elems": ([PP, I32], I64),
         "kx_slot_table": ([PP, I32, I32, P, P], ctypes.c_int),
         "kx_table_fit": ([PP, P, ctypes.POINTER(I32), P], ctypes.c_int),

@@ -673,6 +673,16 @@ extern "C" __attribute__((visibility("hidden"))) int kx_spread_wavelet(
     return launch_spread_d<float, float>(p, a, m, d, st, p->h, work, work_bytes, two_launches);
 }
 
+extern "C" int kx_forward_slots(const kx_plan *p)
+{
+    if (!p || p->abi_version != KX_ABI_VERSION || p->nx <= 0 || p->ny <= 0 || p->nz <= 0 ||
+        p->ntiles <= 0 || p->ns <= 0 || p->nr <= 0 || p->nt < 2)
+        return kx_failf(KX_EINVAL, "forward_slots: bad plan");
+    kx_plan q = *p;
+    q.tabs |= KX_TAB_SLOTS;
+    return pick_slots(&q, q.nh, INT64_MAX, true).rb > 0 || pick_slots(&q, 0, 0, false).rb > 0;
+}
+
 extern "C" __attribute__((visibility("hidden"))) int64_t kx_spread_sums_bytes(const kx_plan *p)
 {
     return (int64_t)pick_slots(p, p->nh, INT64_MAX, true).sums_bytes;

@@ -265,6 +265,21 @@ def make_geom_plan(nx, ny, nz, tile):
     return p
 
 
+# Share of a device's memory that stays free of slot-ordered copies: they are
+# made only while this much is left besides them, so that they never take more
+# than an eighth of the device from what a program could allocate without them
+# (tables of up to an eighth of the device, 36 of 288 GB, have copies).
+SLOTS_FREE = 0.75
+
+
+def slots_affordable(nbytes, device):
+    """Whether copies of ``nbytes`` leave SLOTS_FREE of the device's memory
+    free (memory cached by torch counts as free)."""
+    free, total = torch.cuda.mem_get_info(device)
+    free += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    return free - nbytes >= SLOTS_FREE * total
+
+
 def _empty_table(plan, n, tdt, device, slots):
     """(buffer, view of its (ntiles, n, 64) table): with ``slots`` the buffer
     has room behind the table for its slot-ordered copy."""
@@ -278,6 +293,16 @@ def _fill_slots(plan, n, fmt, buf):
     rc = _lib.load().kx_slot_table(ctypes.byref(plan), n, fmt, _lib.ptr(buf),
                                    _lib.stream_ptr(buf.device))
     _lib.check(rc, "kx_slot_table")
+
+
+def with_slots(plan, tab, fmt):
+    """``tab`` (ntiles, n, 64) copied to a buffer in which its slot-ordered
+    copy follows it."""
+    n = tab.shape[1]
+    buf, out = _empty_table(plan, n, tab.dtype, tab.device, True)
+    out.copy_(tab)
+    _fill_slots(plan, n, fmt, buf)
+    return out
 
 
 def encode(plan, tab, scale, fmt, lo=-math.inf, hi=math.inf, slots=False):

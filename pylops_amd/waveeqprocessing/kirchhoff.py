@@ -261,6 +261,8 @@ class Kirchhoff(LinearOperator):
             object.__setattr__(self, "_dirty", True)
         elif name in _LAUNCH_ATTRS and "_plan" in self.__dict__:
             setattr(self._plan, name, int(value))
+            if name in ("rblock", "sside") and not self._dirty:
+                self._add_slots()
 
     @property
     def itrav(self):
@@ -388,12 +390,15 @@ class Kirchhoff(LinearOperator):
         keep["off_s"], keep["base_s"] = T.encode(plan, ts, inv_dt,
                                                  _lib.KX_F32 if fmt == _lib.KX_F16 else fmt,
                                                  lo_s, hi_s)
-        # float32 operators: the forward's receiver blocks read slot-ordered
-        # copies of the receiver tables
-        slots = self.dtype == np.float32
+        # the forward's receiver blocks read slot-ordered copies of the
+        # receiver tables
+        wfmt = _lib.KX_F64 if self.dtype == np.float64 else _lib.KX_F32
+        plan.dtype, plan.tab_fmt, plan.dynamic = wfmt, fmt, int(self.dynamic)
+        plan.ns, plan.nr, plan.nt, plan.nh = ns, nr, self.nt, len(self.cop.h)
+        plan.rblock, plan.sside = self.rblock, self.sside
+        slots = self._slots_wanted(plan)
         keep["off_r"], keep["base_r"] = T.encode(plan, tr, inv_dt, fmt, lo_r, hi_r, slots)
         del ts, tr
-        wfmt = _lib.KX_F64 if self.dtype == np.float64 else _lib.KX_F32
         if self.dynamic:
             vel = T.as_f64(self.vel, dev).reshape(-1)
             amin, amax = float(self.angleaperture[0]), float(self.angleaperture[1])
@@ -440,21 +445,15 @@ class Kirchhoff(LinearOperator):
                                           device=dev)
             keep["hstar64"] = torch.as_tensor(np.asarray(self.cop.hstar, dtype=np.float64),
                                               device=dev)
-        plan.dtype = wfmt
-        plan.tab_fmt = fmt
-        plan.dynamic = int(self.dynamic)
         if self.dynamic and not bool(keep["izmin"].any()):
             # no trace has an aperture gate: the adjoint skips the test
             plan.dynamic = _lib.KX_DYNAMIC_NOGATE
-        plan.ns, plan.nr, plan.nt = ns, nr, self.nt
         plan.neg_trav = int(neg)
         plan.tabs = _lib.KX_TAB_SLOTS if slots else 0
-        plan.rblock = self.rblock
         plan.sorder = self.sorder
-        plan.sside = self.sside
         plan.gsplit = self.gsplit
         plan.gtiles = self.gtiles
-        plan.nh = keep["h"].numel()
+        assert plan.nh == keep["h"].numel()
         for k, v in keep.items():
             setattr(plan, k, v.data_ptr())
         fit = ctypes.c_int32(0)
@@ -467,6 +466,34 @@ class Kirchhoff(LinearOperator):
         object.__setattr__(self, "_ws_key", None)
         object.__setattr__(self, "_dirty", False)
 
+    def _slots_wanted(self, plan):
+        """Whether the receiver tables get slot-ordered copies: only where a
+        forward of this plan reads them, and while most of the device's
+        memory stays free."""
+        L = _lib.load()
+        wanted = L.kx_forward_slots(ctypes.byref(plan))
+        if wanted <= 0:
+            return False
+        itemsize = 2 if plan.tab_fmt == _lib.KX_F16 else 4
+        nbytes = L.kx_slot_table_elems(ctypes.byref(plan), plan.nr) * itemsize
+        return T.slots_affordable(nbytes * (3 if plan.dynamic else 1), self.device)
+
+    def _add_slots(self):
+        """The copies, for a launch attribute that needs them now.  (The
+        tables they replace stay alive with a batch built on them.)"""
+        plan = self._plan
+        if plan.tabs & _lib.KX_TAB_SLOTS or not self._slots_wanted(plan):
+            return
+        keep = dict(self._dev_tables)
+        for k in ("off_r", "wp_r", "wq_r") if self.dynamic else ("off_r",):
+            keep[k] = T.with_slots(plan, keep[k], _lib.KX_F16 if plan.tab_fmt == _lib.KX_F16
+                                   else _lib.KX_F32)
+        for k, v in keep.items():
+            setattr(plan, k, v.data_ptr())
+        plan.tabs |= _lib.KX_TAB_SLOTS
+        object.__setattr__(self, "_dev_tables", keep)
+        object.__setattr__(self, "_ws_key", None)
+
     @property
     def plan(self):
         """The kx_plan (ctypes) the kernels are launched with."""
@@ -475,15 +502,31 @@ class Kirchhoff(LinearOperator):
         return self._plan
 
     def _work_bytes(self, plan):
-        """Workspace with which the products run fastest, found again when a
+        """Workspace with which the forward runs fastest, found again when a
         launch attribute changed."""
         key = (plan.rblock, plan.sside)
         if getattr(self, "_ws_key", None) != key:
             n = max(int(_lib.load().kx_forward_work_bytes(ctypes.byref(plan))),
-                    self.nsnr * self.nt * self.dtype.itemsize)
+                    self._trace_bytes())
             object.__setattr__(self, "_ws_bytes", n)
             object.__setattr__(self, "_ws_key", key)
         return self._ws_bytes
+
+    def _trace_bytes(self):
+        """Workspace of an adjoint, and the least of a forward."""
+        return self.nsnr * self.nt * self.dtype.itemsize
+
+    def _workspace(self, plan, device, adjoint=False):
+        """Memory for one product: what the forward runs fastest with, or
+        where that much is not to be had, what it needs."""
+        least = self._trace_bytes()
+        nbytes = least if adjoint else self._work_bytes(plan)
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            if nbytes == least:
+                raise
+        return torch.empty(least, dtype=torch.uint8, device=device)
 
     def _product(self, plan, x, out, work, adjoint):
         """Enqueue out <- Op x (Op^H x) on contiguous device tensors."""
@@ -504,9 +547,10 @@ class Kirchhoff(LinearOperator):
         plan = self.plan
         ws = getattr(self, "_ws", None)
         nws = self._work_bytes(plan)
-        if ws is None or ws.numel() < nws or ws.device != x.device:
-            ws = torch.empty(nws, dtype=torch.uint8, device=x.device)
+        if ws is None or self._ws_for < nws or ws.device != x.device:
+            ws = self._workspace(plan, x.device)
             object.__setattr__(self, "_ws", ws)
+            object.__setattr__(self, "_ws_for", nws)
         self._product(plan, x, out, ws, adjoint)
         if adjoint:
             self.rmatvec_count += 1
@@ -518,7 +562,7 @@ class Kirchhoff(LinearOperator):
         plan = self.plan
         xd = to_device(x.reshape(-1), self.dtype, self.device)
         out = torch.empty(nout, dtype=xd.dtype, device=self.device)
-        work = torch.empty(self._work_bytes(plan), dtype=torch.uint8, device=self.device)
+        work = self._workspace(plan, self.device, adjoint)
         self._product(plan, xd, out, work, adjoint)
         return like_input(out, x)
 
