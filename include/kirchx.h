@@ -469,9 +469,15 @@ int kx_eikonal(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, double hx, dou
                double hz, const double *slow, int32_t n, const int32_t *src, double *T,
                int32_t max_iter, int32_t order, int32_t *flag, int32_t *iters, void *stream);
 
-/* kx_eikonal with a workspace of at least kx_eikonal_work_bytes() (0 where
- * none helps: 3D grids, and 2D grids whose shorter side exceeds 1024 cells):
- * every sweep of a source then runs in one launch; the same times and rounds. */
+/* kx_eikonal with a workspace: every sweep of a source then runs in one
+ * launch, as many sources at a time as the workspace holds (at least the
+ * kx_eikonal_work_bytes() of one, else as kx_eikonal).  Each cell is updated
+ * from the same values in the same order; but a source stops by itself, when
+ * its own round changes nothing by more than 1e-13, where kx_eikonal sweeps
+ * on until all have stopped: the times agree to about 1e-12, the rounds are
+ * those of the slowest source.  kx_eikonal_work_bytes() is the size with which
+ * n sources run fastest (0 where none helps: 3D grids, and 2D grids whose
+ * shorter side exceeds 1024 cells). */
 int64_t kx_eikonal_work_bytes(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, int32_t n);
 int kx_eikonal_ws(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, double hx, double hy,
                   double hz, const double *slow, int32_t n, const int32_t *src, double *T,

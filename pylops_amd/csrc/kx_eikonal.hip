@@ -422,10 +422,11 @@ __global__ __launch_bounds__(kSweepThreads) void eik_sweep2d_kernel(EikArgs g,
     }
 }
 
-// T[c * n + s] = W[s * ni + c], 32 x 32 elements per workgroup.
+// T[c * stride + s] = W[s * ni + c] for n tables, 32 x 32 elements per
+// workgroup.
 constexpr int kTr = 32;
 __global__ __launch_bounds__(256) void eik_transpose_kernel(const double *__restrict__ W,
-                                                            int64_t ni, int n,
+                                                            int64_t ni, int n, int stride,
                                                             double *__restrict__ T)
 {
     __shared__ double tile[kTr][kTr + 1];
@@ -437,15 +438,24 @@ __global__ __launch_bounds__(256) void eik_transpose_kernel(const double *__rest
     __syncthreads();
     for (int y = y0; y < kTr; y += 256 / kTr)
         if (s0 + x < n && c0 + y < ni)
-            T[(c0 + y) * n + s0 + x] = tile[x][y];
+            T[(c0 + y) * stride + s0 + x] = tile[x][y];
 }
 
 // Whether a grid's sweeps run in one launch: 2D, the shorter axis one lane
 // per column.
 bool one_launch(int ndims, int nx, int nz, int n)
 {
-    return ndims == 2 && nx > 0 && nz > 0 && n > 0 && std::min(nx, nz) <= kSweepThreads &&
-           n <= 65535 * kTr;
+    return ndims == 2 && nx > 0 && nz > 0 && n > 0 && std::min(nx, nz) <= kSweepThreads;
+}
+
+// Sources whose sweeps can run at once, one workgroup each: more of them take
+// turns, in the same workspace, at no cost (200x200 with 2000 sources 30.3 ms
+// in groups of 512, 32.8 in one; but 301x151 with 600, which all run at once,
+// 14.5 and 9.8 ms).
+int sweep_sources(int nx, int nz)
+{
+    const int threads = (std::min(nx, nz) + 63) & ~63;
+    return 256 * (2048 / threads);  // waves of the chip's 256 CUs
 }
 
 }  // namespace
@@ -456,7 +466,7 @@ extern "C" int64_t kx_eikonal_work_bytes(int32_t ndims, int32_t nx, int32_t ny, 
     (void)ny;
     if (!one_launch(ndims, nx, nz, n))
         return 0;
-    return (int64_t)nx * nz * n * 8 + 64;
+    return (int64_t)nx * nz * std::min(n, sweep_sources(nx, nz)) * 8 + 64;
 }
 
 extern "C" int kx_eikonal(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, double hx, double hy,
@@ -512,10 +522,13 @@ extern "C" int kx_eikonal_ws(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, 
             return efail(KX_ESHAPE, "eikonal: source %d at cell (%d, %d, %d) outside the "
                          "%d x %d x %d grid", k, sx, sy, sz, nx, ny, nz);
     }
-    const int64_t need = kx_eikonal_work_bytes(ndims, nx, ny, nz, n);
-    if (need > 0 && work != nullptr && work_bytes >= need) {
+    const int64_t least = kx_eikonal_work_bytes(ndims, nx, ny, nz, 1);
+    if (least > 0 && work != nullptr && work_bytes >= least) {
+        // as many sources at a time as the workspace holds
+        const int at_once =
+            (int)std::min<int64_t>(std::min(n, sweep_sources(nx, nz)), (work_bytes - 64) / (g.ni * 8));
         double *W = static_cast<double *>(work);
-        int32_t *stat = reinterpret_cast<int32_t *>(W + g.ni * n), h[3] = {0, 0, 0};
+        int32_t *stat = reinterpret_cast<int32_t *>(W + g.ni * at_once), h[3] = {0, 0, 0};
         e = hipMemsetAsync(stat, 0, sizeof(h), st);
         if (e != hipSuccess)
             return efail((int)e, "eikonal: %s", hipGetErrorString(e));
@@ -527,17 +540,20 @@ extern "C" int kx_eikonal_ws(int32_t ndims, int32_t nx, int32_t ny, int32_t nz, 
             if (e != hipSuccess)
                 return efail((int)e, "eikonal: %s", hipGetErrorString(e));
         }
-        hipLaunchKernelGGL(eik_sweep2d_kernel, dim3((unsigned)n), dim3((np + 63) & ~63), lds, st, g, slow, src, W, walk_x,
-                           max_iter, order, stat);
-        e = hipGetLastError();
-        if (e != hipSuccess)
-            return efail((int)e, "eikonal sweeps: %s", hipGetErrorString(e));
-        hipLaunchKernelGGL(eik_transpose_kernel,
-                           dim3((unsigned)((g.ni + kTr - 1) / kTr), (unsigned)((n + kTr - 1) / kTr)),
-                           dim3(256), 0, st, W, g.ni, n, T);
-        e = hipGetLastError();
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(h, stat, sizeof(h), hipMemcpyDeviceToHost, st);
+        for (int s0 = 0; s0 < n; s0 += at_once) {
+            const int ns = std::min(at_once, n - s0);
+            hipLaunchKernelGGL(eik_sweep2d_kernel, dim3((unsigned)ns), dim3((np + 63) & ~63), lds,
+                               st, g, slow, src + 3 * (int64_t)s0, W, walk_x, max_iter, order,
+                               stat);
+            hipLaunchKernelGGL(eik_transpose_kernel,
+                               dim3((unsigned)((g.ni + kTr - 1) / kTr),
+                                    (unsigned)((ns + kTr - 1) / kTr)),
+                               dim3(256), 0, st, W, g.ni, ns, n, T + s0);
+            e = hipGetLastError();
+            if (e != hipSuccess)
+                return efail((int)e, "eikonal sweeps: %s", hipGetErrorString(e));
+        }
+        e = hipMemcpyAsync(h, stat, sizeof(h), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess)
             e = hipStreamSynchronize(st);
         if (e != hipSuccess)

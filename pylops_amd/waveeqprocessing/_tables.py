@@ -105,9 +105,9 @@ def eikonal(pts, vel, origin, dsamp, dims, device, unit=False, max_iter=20, orde
     iters = (ctypes.c_int32 * 2)(0, 0)
     L = _lib.load()
     slow = slow.contiguous()
-    # room for the sweeps of a 2D grid to run in one launch
-    work = torch.empty(L.kx_eikonal_work_bytes(ndims, nx, ny, nz, n), dtype=torch.uint8,
-                       device=device)
+    # room for the sweeps of a 2D grid to run in one launch: for all tables,
+    # or as many as memory is left for besides them
+    work = _eikonal_work(n, lambda k: L.kx_eikonal_work_bytes(ndims, nx, ny, nz, k), device)
     rc = L.kx_eikonal_ws(ndims, nx, ny, nz, hx, hy, hz, _lib.ptr(slow), n, _lib.ptr(srcd),
                          _lib.ptr(out), max_iter, order, _lib.ptr(flag), iters,
                          _lib.ptr(work) if work.numel() else None, work.numel(),
@@ -119,6 +119,19 @@ def eikonal(pts, vel, origin, dsamp, dims, device, unit=False, max_iter=20, orde
             f"eikonal traveltimes did not converge in {max_iter} sweep rounds per phase "
             f"({iters[0]} rounds run); pass a larger eikonal_iter")
     return out
+
+
+def _eikonal_work(n, nbytes, device):
+    """A workspace for the largest number of tables, n or a half of it and so
+    on, that can be allocated; none below 64 (or n) of them, where one launch
+    per anti-diagonal for all tables is as fast."""
+    k = n
+    while k >= min(n, 64):
+        try:
+            return torch.empty(nbytes(k), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            k //= 2
+    return torch.empty(0, dtype=torch.uint8, device=device)
 
 
 def eikonal_tables(srcs, recs, vel, origin, dsamp, dims, device, distances, max_iter=20):
