@@ -5,19 +5,21 @@ change their results beyond rounding (the float32 forward not at all):
 
 - ``tile`` (tz, tx, ty), the image block of one wavefront (the tables are
   rebuilt for each candidate);
-- ``rblock``, receivers (or sources) per forward workgroup, ``sorder``,
-  the forward's lane order, and ``sside``, which side a forward workgroup
-  blocks (single problems);
+- ``rblock``, receivers (or sources) per forward workgroup, and for blocks
+  of 4, 2 and 1 ``sorder``, the forward's lane order, and ``sside``, which
+  side a forward workgroup blocks (single problems; blocks of 8 and 16 hold
+  receivers in an order of their own);
 - ``gsplit``, adjoint waves per tile.
 
 :func:`autotune` times every candidate on the device with a dense random
 model (every tile busy, as in solver iterations after the first) and
-returns the fastest; :func:`autotune_batch` does the same for a batch,
+returns the fastest, timing the products as an operator runs them, with
+their wavelet and workspace; :func:`autotune_batch` does the same for a batch,
 where the tile applies to every problem and the other three to the batch's
 persistent launches.  The forward and adjoint are tuned independently for
 each tile (their shapes do not interact); the tile with the smallest sum
-wins.  Results are kept in a JSON cache keyed by geometry, precision and
-device name.
+wins.  Results are kept in a JSON cache keyed by the generation of the
+kernels, geometry, wavelet length, precision and device name.
 """
 import ctypes
 import json
@@ -34,6 +36,9 @@ __all__ = ["autotune", "autotune_batch", "TILES_2D", "TILES_3D"]
 TILES_2D = ((16, 4, 1), (8, 8, 1), (32, 2, 1), (4, 16, 1))
 TILES_3D = ((16, 2, 2), (8, 4, 2), (4, 4, 4), (8, 8, 1), (16, 4, 1))
 RBLOCKS = (16, 8, 4, 2, 1)
+# part of the cache key: raised when the kernels or the launch rules change, so
+# that shapes measured with earlier ones are measured again
+KERNELS = 2
 SORDERS = (_lib.KX_ORDER_NATURAL, _lib.KX_ORDER_ROTATED)
 SSIDES = (_lib.KX_SIDE_RECEIVERS, _lib.KX_SIDE_SOURCES)
 GSPLITS = (1, 2, 4)
@@ -86,8 +91,9 @@ def _key(kind, kws, device):
     for kw in kws:
         g = _geometry(kw)
         parts.append("x".join(str(v) for v in g) + f":{int(bool(kw.get('dynamic', False)))}"
-                     f":{kw.get('dtype', 'float64')}:{kw.get('tabledtype')}")
-    return f"{kind}|{dev}|" + ";".join(parts)
+                     f":{kw.get('dtype', 'float64')}:{kw.get('tabledtype')}"
+                     f":w{len(kw['wav'])}")
+    return f"{kind}|k{KERNELS}|{dev}|" + ";".join(parts)
 
 
 def _timer(fn, reps):
@@ -102,25 +108,42 @@ def _timer(fn, reps):
     return a.elapsed_time(b) / reps
 
 
-def _candidates_fwd(dtype, dynamic, nt, sides=(_lib.KX_SIDE_RECEIVERS,), orders=SORDERS,
-                    lds=65536):
-    max_rb = 4 if dtype == "float64" else (8 if dynamic else 16)
-    if dtype == "float64":
-        sides = (_lib.KX_SIDE_RECEIVERS,)  # float64 operators block receivers
-    for rb in RBLOCKS:
-        # the forward's LDS rows: nt rounded up to 2 mod 16 samples of 8 bytes
-        if rb > max_rb or (rb > 1 and rb * (nt + (2 - nt) % 16) * 8 > lds):
-            continue  # more registers than two workgroups per CU, or LDS
-        for so in orders if rb > 1 else (_lib.KX_ORDER_NATURAL,):
-            for side in sides:
+def _rows_fit(rb, nt, lds):
+    # the forward's LDS rows: nt rounded up to 2 mod 16 samples of 8 bytes
+    return rb == 1 or rb * (nt + (2 - nt) % 16) * 8 <= lds
+
+
+def _candidates_fwd(dtype, nt, nr, lds):
+    """(rblock, sorder, sside) of an operator's forward."""
+    if dtype != "float64":
+        # blocks of 16 and 8: one launch each, whatever the order (with up to
+        # 8 receivers half of a block of 16 would stay empty)
+        for rb in (16, 8):
+            if rb * nt * 8 <= lds and rb < 2 * max(nr, 5):
+                yield rb, _lib.KX_ORDER_NATURAL, _lib.KX_SIDE_RECEIVERS
+    for rb in (4, 2, 1):
+        if not _rows_fit(rb, nt, lds):
+            continue
+        for so in SORDERS if rb > 1 else (_lib.KX_ORDER_NATURAL,):
+            # float64 operators block receivers
+            for side in SSIDES if dtype != "float64" else (_lib.KX_SIDE_RECEIVERS,):
                 yield rb, so, side
+
+
+def _candidates_batch(dtype, dynamic, nt, lds=65536):
+    """(rblock, sorder) of a batch's forward."""
+    max_rb = 4 if dtype == "float64" else (8 if dynamic else 16)
+    for rb in RBLOCKS:
+        if rb <= max_rb and _rows_fit(rb, nt, lds):
+            for so in SORDERS if rb > 1 else (_lib.KX_ORDER_NATURAL,):
+                yield rb, so
 
 
 def autotune(reps=3, tiles=None, cache=None, **kw):
     """Fastest launch shapes for ``Kirchhoff(**kw)``: returns a dict with
     ``tile``, ``rblock``, ``sorder``, ``sside``, ``gsplit``, ``gtiles``
-    (pass it on to ``Kirchhoff``) and the measured ``ms`` (forward kernel +
-    adjoint kernel).  ``tiles`` overrides the candidate tiles; ``cache`` is the
+    (pass it on to ``Kirchhoff``) and the measured ``ms`` (forward +
+    adjoint).  ``tiles`` overrides the candidate tiles; ``cache`` is the
     JSON cache file (default ``$PYLOPS_AMD_TUNE_CACHE`` or
     ``~/.cache/pylops_amd/tune.json``; ``False`` disables it)."""
     from pylops_amd.waveeqprocessing.kirchhoff import Kirchhoff
@@ -134,8 +157,6 @@ def autotune(reps=3, tiles=None, cache=None, **kw):
         hit = _load(path).get(key)
         if hit is not None:
             hit["tile"] = tuple(hit["tile"])
-            hit.setdefault("sside", _lib.KX_SIDE_AUTO)  # entries from before sside was tuned
-            hit.setdefault("gtiles", 0)  # entries from before gtiles was tuned
             return hit
     ndims = _geometry(kw)[0]
     tiles = tiles or (TILES_2D if ndims == 2 else TILES_3D)
@@ -147,33 +168,34 @@ def autotune(reps=3, tiles=None, cache=None, **kw):
         if tile[0] > len(kw["z"]) * 2:
             continue  # a tile twice as tall as the image wastes lanes
         Op = Kirchhoff(**kw, tile=tile)
-        plan = Op.plan
         g = torch.Generator(device="cpu").manual_seed(0)
         m = torch.randn(Op.ni, generator=g, dtype=tdt).to(Op.device)
         traces = torch.empty(Op.nsnr * Op.nt, dtype=tdt, device=Op.device)
         img = torch.empty(Op.ni, dtype=tdt, device=Op.device)
-        st = _lib.stream_ptr(Op.device)
-        L.kx_spread(ctypes.byref(plan), _lib.ptr(m), _lib.ptr(traces), st)
 
-        def spread():
-            _lib.check(L.kx_spread(ctypes.byref(plan), _lib.ptr(m), _lib.ptr(traces), st),
-                       "kx_spread")
+        def forward():
+            if Op._fwd_dtype != Op.dtype:  # convolved apart, in float64
+                _lib.check(L.kx_spread(ctypes.byref(Op.plan), _lib.ptr(m), _lib.ptr(traces),
+                                       _lib.stream_ptr(Op.device)), "kx_spread")
+            else:
+                Op._into(m, traces, False)
 
-        def gather():
-            _lib.check(L.kx_gather(ctypes.byref(plan), _lib.ptr(traces), _lib.ptr(img), st),
-                       "kx_gather")
+        def adjoint():
+            Op._into(traces, img, True)
 
         fwd = []
         lds = torch.cuda.get_device_properties(Op.device).shared_memory_per_block
-        for rb, so, side in _candidates_fwd(dtype, kw.get("dynamic", False), len(kw["t"]),
-                                            SSIDES, lds=lds):
-            plan.rblock, plan.sorder, plan.sside = rb, so, side
-            fwd.append((_timer(spread, reps), rb, so, side))
+        for rb, so, side in _candidates_fwd(dtype, len(kw["t"]), Op.nsnr if not Op.travsrcrec
+                                            else Op.nr, lds):
+            Op.rblock, Op.sorder, Op.sside = rb, so, side
+            if rb > 4 and not Op.plan.tabs & _lib.KX_TAB_SLOTS:
+                continue  # no memory for the tables of such blocks
+            fwd.append((_timer(forward, reps), rb, so, side))
         adj = []
         for gs in GSPLITS:
             for gt in GTILES:
-                plan.gsplit, plan.gtiles = gs, gt
-                adj.append((_timer(gather, reps), gs, gt))
+                Op.gsplit, Op.gtiles = gs, gt
+                adj.append((_timer(adjoint, reps), gs, gt))
         tf, rb, so, side = min(fwd)
         ta, gs, gt = min(adj)
         cand = {"tile": tuple(tile), "rblock": rb, "sorder": so, "sside": side, "gsplit": gs,
@@ -206,7 +228,6 @@ def autotune_batch(kws, reps=3, tiles=None, cache=None):
         hit = _load(path).get(key)
         if hit is not None:
             hit["tile"] = tuple(hit["tile"])
-            hit.setdefault("gtiles", 0)  # entries from before gtiles was tuned
             return hit
     ndims = _geometry(kws[0])[0]
     tiles = tiles or (TILES_2D if ndims == 2 else TILES_3D)
@@ -223,9 +244,7 @@ def autotune_batch(kws, reps=3, tiles=None, cache=None):
         a = torch.empty(B0.shape[1], dtype=tdt, device=B0.device)
         B0._into(m, d, False)
         fwd = []
-        for rb, so, _ in _candidates_fwd(dtype, dynamic, max(len(kw["t"]) for kw in kws),
-                                         orders=(_lib.KX_ORDER_NATURAL,
-                                                 _lib.KX_ORDER_ROTATED)):
+        for rb, so in _candidates_batch(dtype, dynamic, max(len(kw["t"]) for kw in kws)):
             B = KirchhoffBatch(ops, rblock=rb, sorder=so)
             if B.rblock != rb:
                 continue  # does not fit the batch's longest trace
