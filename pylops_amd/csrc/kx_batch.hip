@@ -274,17 +274,6 @@ struct Layout {
     int64_t n_spread, n_gather, n_conv;
 };
 
-int device_cus()
-{
-    int cus = 256, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-        (void)hipGetLastError();
-        cus = 256;
-    }
-    return cus;
-}
-
 // Largest receiver block per element type: registers per lane grow with the
 // block, and two workgroups per CU are kept.
 template <typename TD, bool DYN> constexpr int max_rblock()

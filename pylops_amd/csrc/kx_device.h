@@ -6,6 +6,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <type_traits>
 
@@ -20,27 +21,40 @@ constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kLdsBudget = 64 * 1024;  // LDS of one workgroup on every CDNA device
 
-// LDS one workgroup of the current device may use: the device's limit
-// (160 KB on gfx950), queried once per device, or kLdsBudget without one.
-inline size_t lds_budget()
+// An attribute of the current device, looked up once per device (a launch asks
+// for several of them); `without` when there is no device or it reports less
+// than `least`.
+template <hipDeviceAttribute_t ATTR> int device_attribute(int without, int least)
 {
-    static int cached[64] = {};
+    static std::atomic<int> cached[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
         (void)hipGetLastError();
-        return kLdsBudget;
+        return without;
     }
-    if (cached[dev] == 0) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) !=
-                hipSuccess ||
-            v < kLdsBudget) {
+    int v = cached[dev].load(std::memory_order_relaxed);
+    if (v == 0) {
+        if (hipDeviceGetAttribute(&v, ATTR, dev) != hipSuccess || v < least) {
             (void)hipGetLastError();
-            v = kLdsBudget;
+            v = without;
         }
-        cached[dev] = v;
+        cached[dev].store(v, std::memory_order_relaxed);
     }
-    return (size_t)cached[dev];
+    return v;
+}
+
+// LDS one workgroup of the current device may use: the device's limit
+// (160 KB on gfx950), or kLdsBudget without one.
+inline size_t lds_budget()
+{
+    return (size_t)device_attribute<hipDeviceAttributeMaxSharedMemoryPerBlock>(kLdsBudget,
+                                                                              kLdsBudget);
+}
+
+// Compute units of the current device.
+inline int device_cus()
+{
+    return device_attribute<hipDeviceAttributeMultiprocessorCount>(256, 1);
 }
 
 // Lets kernel fn take `lds` bytes of dynamic LDS (beyond 64 KB the

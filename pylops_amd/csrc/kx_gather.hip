@@ -26,17 +26,6 @@ __global__ __launch_bounds__(kGatherBlock) void gather_kernel(KArgs a, const TD 
                                                        dstride, mstride);
 }
 
-int device_cus()
-{
-    int cus = 256, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-        (void)hipGetLastError();
-        cus = 256;
-    }
-    return cus;
-}
-
 // the same for plans whose samples all lie in their windows
 template <typename TD, typename TT, bool DYN, int JW, int P, int NP, int K, bool GATE>
 __global__ __launch_bounds__(kGatherBlock, (FitWaves<TD, DYN, NP, K>::v)) void gather_fit_kernel(

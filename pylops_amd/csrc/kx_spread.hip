@@ -156,17 +156,6 @@ __global__ __launch_bounds__(kSpreadBlock) void spread_models_kernel(
 
 constexpr int kRblocks[] = {4, 2, 1};
 
-int device_cus()
-{
-    int cus = 256, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-        (void)hipGetLastError();
-        cus = 256;
-    }
-    return cus;
-}
-
 constexpr int kLdsPerCu = 160 * 1024;
 constexpr int kMaxWavesPerCu = 32;
 
