@@ -536,8 +536,8 @@ extern "C" int kx_conv_rows(const void *x, int64_t xstride, void *y, int64_t ntr
     const int nseg = (nt + kConvOut - 1) / kConvOut;
     if (ntr * nseg > INT32_MAX)
         return kx_fail(KX_ESHAPE, "conv: too many traces");
-    const size_t lds = (size_t)conv_lds_elems(nh) * (dtype == KX_F64 ? 8 : 4);
-    if (lds > (size_t)kLdsBudget)
+    const size_t es = dtype == KX_F64 ? 8 : 4, lds = (size_t)conv_lds_elems(nh) * es;
+    if (conv_lds_limit_elems(nh) * es > (size_t)kLdsBudget)
         return kx_fail(KX_ELDS, "conv: filter of %d taps does not fit LDS", nh);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const dim3 grid((unsigned)(ntr * nseg));

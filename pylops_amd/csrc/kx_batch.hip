@@ -459,7 +459,7 @@ int check_batch(const kx_plan *plans, int nprob)
             return bfail(KX_ELDS, "batch: problem %d: nt=%d does not fit one trace in LDS "
                                   "(the single-problem operator spreads such traces in time "
                                   "segments)", p, a.nt);
-        const size_t clds = (size_t)conv_lds_elems(a.nh) * dsize(a.dtype);
+        const size_t clds = conv_lds_limit_elems(a.nh) * dsize(a.dtype);
         if (clds > (size_t)kLdsBudget)
             return bfail(KX_ELDS, "batch: problem %d: filter of %d taps does not fit LDS", p,
                          a.nh);

@@ -1597,12 +1597,20 @@ __device__ __forceinline__ void gather_tiles(const KArgs &a, const TD *__restric
 // loads).  Long filters of float32 data take 32 taps at a time (LONG, a kernel
 // of its own: with both loops in one the compiler made the shorter 1.6 times
 // slower): 300 traces of 64 samples, 1001 taps, 21.1 and 19.1 us.
+constexpr int kConvChunk = 16;
+
 // LDS elements of one convolution workgroup: window + one group of
-// read-ahead, and the filter's length once more (the taps of a short filter;
-// it also keeps the longest filter accepted what it was while all were staged)
+// read-ahead, and the taps of a short filter.
 __host__ __device__ __forceinline__ int conv_lds_elems(int nh)
 {
-    return conv_taps_padded(nh) + kConvOut + conv_taps_padded(nh) + 4;
+    const int nhp = conv_taps_padded(nh);
+    return kConvOut + nhp + 4 + (nhp < kConvChunk ? nhp : kConvChunk);
+}
+// What the longest filter accepted is measured by: the window with all taps
+// beside it.
+inline size_t conv_lds_limit_elems(int nh)
+{
+    return (size_t)kConvOut + 2 * (size_t)conv_taps_padded(nh) + 4;
 }
 
 // adjacent samples in LDS (aligned), and of a row of y (which is not)
@@ -1641,7 +1649,7 @@ __device__ __forceinline__ void conv_segment(const TD *__restrict__ x, int64_t x
     for (int q = 0; q < kAhead; ++q)
         ahead[q] = xr[min(max(start + q * kConvThreads + (int)threadIdx.x, 0), nt - 1)];
     TD *hs = win + nwin;  // the taps of a filter without a chunk, flipped
-    constexpr int kChunk = 16;
+    constexpr int kChunk = kConvChunk;
     if (!LONG && nh < kChunk && (int)threadIdx.x < nhp)
         hs[threadIdx.x] = (int)threadIdx.x < nh ? h[tr * hstride + nh - 1 - threadIdx.x] : TD(0);
 #pragma unroll

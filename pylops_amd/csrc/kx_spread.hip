@@ -217,11 +217,9 @@ int spread_per_cu(const void *fn, int rb, int nt)
 // can hide the latency of the table loads; ties go to the larger block,
 // which re-reads the image and the source table less often.
 template <typename TD, typename TT, bool DYN, bool NEG, bool XS, int ORD>
-int pick_rblock(int requested, int nr, int nt, int max_rb)
+int pick_rblock(int requested, int nr, int nt)
 {
-    auto fits = [&](int rb) {
-        return rb <= max_rb && spread_lds_bytes(rb, nt) <= lds_budget();
-    };
+    auto fits = [&](int rb) { return spread_lds_bytes(rb, nt) <= lds_budget(); };
     if (requested > 0) {
         for (int rb : kRblocks)
             if (rb <= requested && fits(rb))
@@ -246,10 +244,10 @@ int pick_rblock(int requested, int nr, int nt, int max_rb)
 }
 
 template <typename TD, typename TT, bool DYN, bool NEG, bool XS, int ORD>
-int launch_spread_o(KArgs a, int requested, int max_rb, const void *m, void *y,
-                    const SpreadScale *sc, hipStream_t st, const void *h, int nh)
+int launch_spread_o(KArgs a, int requested, const void *m, void *y, const SpreadScale *sc,
+                     hipStream_t st, const void *h, int nh)
 {
-    a.rblock = pick_rblock<TD, TT, DYN, NEG, XS, ORD>(requested, a.nr, a.nt, max_rb);
+    a.rblock = pick_rblock<TD, TT, DYN, NEG, XS, ORD>(requested, a.nr, a.nt);
     switch (a.rblock) {
     case 4:
         return launch_spread_rb<TD, TT, DYN, NEG, XS, ORD, 4>(a, m, y, sc, st, h, nh);
@@ -494,16 +492,16 @@ int launch_slots_d(const kx_plan *p, const KArgs &a, const SlotsShape &g, const 
 }
 
 template <typename TD, typename TT, bool DYN, bool NEG, bool XS>
-int launch_spread_t(const KArgs &a, int order, int requested, int max_rb, const void *m, void *y,
+int launch_spread_t(const KArgs &a, int order, int requested, const void *m, void *y,
                     const SpreadScale *sc, hipStream_t st, const void *h, int nh)
 {
     switch (order) {
     case KX_ORDER_ROTATED:
-        return launch_spread_o<TD, TT, DYN, NEG, XS, kOrdRotated>(a, requested, max_rb, m, y,
-                                                                  sc, st, h, nh);
+        return launch_spread_o<TD, TT, DYN, NEG, XS, kOrdRotated>(a, requested, m, y, sc, st, h,
+                                                                  nh);
     default:
-        return launch_spread_o<TD, TT, DYN, NEG, XS, kOrdNatural>(a, requested, max_rb, m, y,
-                                                                  sc, st, h, nh);
+        return launch_spread_o<TD, TT, DYN, NEG, XS, kOrdNatural>(a, requested, m, y, sc, st, h,
+                                                                  nh);
     }
 }
 
@@ -558,8 +556,6 @@ int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream
         return KX_ENOFUSE;
     if (sizeof(TD) == 4 && !p->aux)
         return kx_failf(KX_EINVAL, "spread: plan.aux (KX_AUX_BYTES of device scratch) is NULL");
-    // registers per lane grow with the block: keep two workgroups per CU
-    const int max_rb = 4;
     SpreadScale *sc = reinterpret_cast<SpreadScale *>(p->aux);
     const SlotsShape slots = pick_slots(p, nh, work ? work_bytes : 0, two_launches);
     if (slots.rb && h != nullptr && !slots.fused)
@@ -587,12 +583,13 @@ int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream
     // transposed positions: T = os + or and the integer bases add in either
     // order, and the dynamic kernel (XS) forms the source-side products per
     // step, so the traces are bitwise those of blocks of receivers.
-    // Automatic: a 2D plan blocks the side with fewer members, whose rows
-    // then serve many workgroups through L2 (on a 61 x 301 geometry 13%
-    // faster kinematic, either way round, and 6% with dynamic weights: 3.68
-    // against 3.91 ms for the forward with its wavelet); 3D plans block
-    // receivers (measured slower otherwise: 128x128x120 with 25 x 400, 24.2
-    // against 22.8 ms for the natural order, 17.4 against 15.8 ms rotated).
+    // Automatic, where the plan takes no slot blocks: a 2D plan blocks the
+    // side with fewer members, whose rows then serve many workgroups through
+    // L2 (on a 61 x 301 geometry 13% faster kinematic, either way round, and
+    // 6% with dynamic weights: 3.68 against 3.91 ms for the forward with its
+    // wavelet); 3D plans block receivers (measured slower otherwise:
+    // 128x128x120 with 25 x 400, 24.2 against 22.8 ms for the natural order,
+    // 17.4 against 15.8 ms rotated).
     if (seg)
         return p->dynamic ? (p->neg_trav ? launch_spread_seg<TD, TT, true, true>(a, m, y, sc, st)
                                          : launch_spread_seg<TD, TT, true, false>(a, m, y, sc, st))
@@ -610,20 +607,18 @@ int launch_spread_d(const kx_plan *p, KArgs a, const void *m, void *y, hipStream
     // exchanged-side dynamic kernels exist for float32 operators only (xs
     // is false otherwise)
     constexpr bool kXS = sizeof(TD) == 4;
+    const int rb = p->rblock;
     if (p->dynamic && xs)
-        return p->neg_trav ? launch_spread_t<TD, TT, true, true, kXS>(a, order, p->rblock, max_rb,
-                                                                      m, y, sc, st, h, nh)
-                           : launch_spread_t<TD, TT, true, false, kXS>(a, order, p->rblock,
-                                                                       max_rb, m, y, sc, st, h, nh);
+        return p->neg_trav
+                   ? launch_spread_t<TD, TT, true, true, kXS>(a, order, rb, m, y, sc, st, h, nh)
+                   : launch_spread_t<TD, TT, true, false, kXS>(a, order, rb, m, y, sc, st, h, nh);
     if (p->dynamic)
-        return p->neg_trav ? launch_spread_t<TD, TT, true, true, false>(a, order, p->rblock,
-                                                                        max_rb, m, y, sc, st, h, nh)
-                           : launch_spread_t<TD, TT, true, false, false>(a, order, p->rblock,
-                                                                         max_rb, m, y, sc, st, h, nh);
-    return p->neg_trav ? launch_spread_t<TD, TT, false, true, false>(a, order, p->rblock, max_rb,
-                                                                     m, y, sc, st, h, nh)
-                       : launch_spread_t<TD, TT, false, false, false>(a, order, p->rblock,
-                                                                      max_rb, m, y, sc, st, h, nh);
+        return p->neg_trav
+                   ? launch_spread_t<TD, TT, true, true, false>(a, order, rb, m, y, sc, st, h, nh)
+                   : launch_spread_t<TD, TT, true, false, false>(a, order, rb, m, y, sc, st, h, nh);
+    return p->neg_trav
+               ? launch_spread_t<TD, TT, false, true, false>(a, order, rb, m, y, sc, st, h, nh)
+               : launch_spread_t<TD, TT, false, false, false>(a, order, rb, m, y, sc, st, h, nh);
 }
 
 }  // namespace
