@@ -289,6 +289,10 @@ def slots_affordable(nbytes, device):
     """Whether copies of ``nbytes`` leave SLOTS_FREE of the device's memory
     free (memory cached by torch counts as free)."""
     free, total = torch.cuda.mem_get_info(device)
+    if free - nbytes >= SLOTS_FREE * total:
+        return True
+    # (asked only now: torch's statistics take longer than a small operator's
+    # tables)
     free += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
     return free - nbytes >= SLOTS_FREE * total
 
