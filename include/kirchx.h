@@ -122,9 +122,13 @@ typedef struct kx_plan {
     int32_t ntz, ntx, nty;
     int64_t ntiles;      /* ntz*ntx*nty */
     int32_t neg_trav;    /* 1 if a traveltime may be negative (truncation path) */
-    int32_t rblock;      /* receivers (sources, see sside) per spread workgroup, 0 = automatic */
+    int32_t rblock;      /* at most so many receivers (sources, see sside) per
+                            spread workgroup, 0 = automatic.  8 and 16: slot
+                            blocks of receivers, with KX_TAB_SLOTS and unless
+                            sside asks for sources; otherwise 4, 2 and 1 */
     int32_t nh;          /* wavelet length after offset padding (odd) */
-    int32_t sorder;      /* spread lane order KX_ORDER_*, 0 = automatic */
+    int32_t sorder;      /* lane order KX_ORDER_* of blocks of 4 and 2, 0 =
+                            automatic (slot blocks have an order of their own) */
     const void *off_s;
     const int32_t *base_s;
     const void *off_r;
@@ -140,7 +144,9 @@ typedef struct kx_plan {
                      share one aux must be ordered on one stream */
     int32_t gsplit; /* waves per tile in the adjoint, 1, 2 or 4 (each sums a
                        share of the sources), 0 = automatic */
-    int32_t sside;  /* forward workgroup blocks KX_SIDE_*, 0 = automatic */
+    int32_t sside;  /* what a forward workgroup blocks, KX_SIDE_*; 0 = slot
+                       blocks of receivers where they are the faster, otherwise
+                       in 2D the side with fewer members (float32 tables) */
     int32_t gtiles; /* neighbouring image tiles per wave in the adjoint (1, 2
                        or 4; they share the staged trace windows),
                        0 = automatic */
@@ -260,7 +266,7 @@ int kx_forward(const kx_plan *p, const void *m, void *d, void *work, void *strea
  * shares the image tiles of a block between several workgroups, each keeping
  * its 64-bit sums in the workspace, and adds them in a second launch (the
  * data are bitwise the same).  kx_forward_work_bytes() is the size with which
- * it runs fastest. */
+ * it runs fastest (up to 0.7 GB more than the traces).  work: 8-byte aligned. */
 int64_t kx_forward_work_bytes(const kx_plan *p);
 int kx_forward_ws(const kx_plan *p, const void *m, void *d, void *work, int64_t work_bytes,
                   void *stream);

@@ -250,8 +250,9 @@ __global__ __launch_bounds__(kEikBlock) void eik_sweep_kernel(EikArgs g,
 constexpr int kAhead = 8;
 constexpr int kSweepThreads = 1024;
 
-// x / 3 as a division rounds it, in three operations (|x| well inside the
-// normal range: times, and 1e30 for none).
+// x / 3 as a division rounds it, in three operations: the product with the
+// rounded reciprocal, corrected by its fused residual (Markstein's correction
+// of a quotient; |x| well inside the normal range: times, and 1e30 for none).
 __device__ __forceinline__ double third(double x)
 {
     const double r = 1.0 / 3.0, q = x * r;

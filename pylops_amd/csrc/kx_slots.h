@@ -24,15 +24,15 @@ namespace {
 // (RB = 8).  The receiver's entries of the RB points come from the
 // slot-ordered copy of the table: 16-byte loads, contiguous over the lanes
 // (read from the tiled table, 64 row parts per instruction, the 3D kernel
-// took 18.8 ms instead of 12.4 ms).  A receiver's base is one value per lane
+// took 18.8 ms where this order first took 12.4).  A receiver's base is one value per lane
 // and tile.  A step is 11 (kinematic, RB = 16) to 17 (dynamic, RB = 8) vector
 // instructions and two atomics, against about 17 and 20 with rows one after
 // the other.
 // Measured, forward with its wavelet: 3D 128x128x120 with 25 x 400, kinematic
-// float32 15.8 to 10.0 ms (16.4 clocks of a CU per step; the vector
+// float32 15.7 to 10.4 ms (16.4 clocks of a CU per step; the vector
 // instructions and the atomics take about 12 each, and either alone with the
 // loads 13 to 14); 3D 93x77x101 with 12 x 195, float16 tables, 1.89 to 1.12
-// ms; 2D 601x300 with 61 x 301, dynamic float32, RB = 8, 3.58 to 3.49 ms:
+// ms; 2D 601x300 with 61 x 301, dynamic float32, RB = 8, 3.58 to 3.54 ms:
 // bound by its loads (12 bytes per triplet through L1; without them 2.0 ms,
 // without the atomics 3.5 ms).
 constexpr int kSlotsMaxThreads = 1024;

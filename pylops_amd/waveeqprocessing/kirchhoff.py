@@ -83,10 +83,13 @@ class Kirchhoff(LinearOperator):
         dtype.
     tile : ``(tz, tx, ty)`` image tile of 64 points.
     device : torch device of the tables (default: current HIP device).
-    rblock : receivers (or sources, see ``sside``) per forward workgroup
-        (0 = automatic).
-    sorder : forward lane order, ``KX_ORDER_NATURAL`` (1) or
-        ``KX_ORDER_ROTATED`` (2); 0 = automatic.
+    rblock : receivers (or sources, see ``sside``) per forward workgroup at
+        most (0 = automatic).  Blocks of 8 and 16 (float32 operators,
+        receivers) read a second, slot-ordered copy of the receiver tables,
+        made where the automatic choice or this one needs it and while three
+        quarters of the device's memory stay free.
+    sorder : forward lane order of blocks of 4 and 2, ``KX_ORDER_NATURAL`` (1)
+        or ``KX_ORDER_ROTATED`` (2); 0 = automatic.
     gsplit : adjoint waves per tile group, 1, 2 or 4; 0 = automatic.
     gtiles : neighbouring image tiles per adjoint wave, sharing its staged
         trace windows, 1, 2 or 4; 0 = automatic.
@@ -95,8 +98,8 @@ class Kirchhoff(LinearOperator):
         ``RuntimeError``.
     sside : what a forward workgroup blocks, ``KX_SIDE_RECEIVERS`` (1: one
         source, a block of receivers) or ``KX_SIDE_SOURCES`` (2: one
-        receiver, a block of sources; float32 operators); 0 = automatic.
-        Every choice gives bitwise the same data.
+        receiver, a block of at most 4 sources; float32 operators); 0 =
+        automatic.  Every choice gives bitwise the same data.
 
     ``waveeqprocessing.autotune`` measures the fastest ``tile``, ``rblock``,
     ``sorder``, ``sside`` and ``gsplit`` for a geometry.
