@@ -278,9 +278,9 @@ struct SlotsShape {
 };
 
 // Estimated times of a forward, in microseconds: sums of terms whose factors
-// were fitted to the measured times of 579 random 2D and 3D operators (64 to
-// 5000 tiles, 1 to 61 sources, 2 to 400 receivers, 200 to 2500 samples, 41 to
-// 2400 taps; 9300 launches, 90% of them within 12%).
+// were fitted to the measured times of 1859 random 2D and 3D operators (2 to
+// 13000 tiles, 1 to 61 sources, 2 to 400 receivers, 60 to 2500 samples, 41 to
+// 2300 taps; 27800 launches, 80% of them within 15%).
 //   fixed   the launches
 //   round   a round of workgroups
 //   clear   clearing and writing out, per 1000 samples of a CU
@@ -299,18 +299,18 @@ struct SlotsTime {
     double add_conv;  // ... its convolution, per 1000 four-tap steps of a thread
 };
 constexpr RowsTime kRowsTime[2] = {  // kinematic, dynamic
-    {7.35, 0.63, 7.97, 12.3, 10.5, 248.0},
-    {8.87, 0.57, 10.3, 2.3, 11.7, 280.0},
+    {7.17, 0.329, 8.65, 11.5, 11.2, 228.0},
+    {8.05, 0.356, 10.8, 0.0, 11.4, 277.0},
 };
 constexpr SlotsTime kSlotsTime[2][2][2] = {  // [dynamic][blocks of 16][1024 threads]
-    {{{10.8, 0, 0, 4.73, 71.1, 12.7, 36.9, 0.342, 75.4},
-      {11.8, 2.14, 0, 11.7, 0, 10.3, 38.3, 0.309, 55.3}},
-     {{10.4, 0, 0.0234, 4.13, 43.7, 9.91, 35.7, 0.52, 78.2},
-      {5, 7.68, 0.066, 7.89, 0, 9.49, 35, 0.309, 73.5}}},
-    {{{10.9, 0.757, 0.0304, 7.87, 47.6, 14.6, 35.3, 0.344, 71.8},
-      {8.18, 3.28, 0.251, 11.3, 0, 16.1, 36.5, 0.172, 67.7}},
-     {{10.6, 0, 0.125, 6.42, 37.2, 12.4, 33.7, 0.479, 76.8},
-      {3.06, 6.75, 0.256, 9.03, 0, 10.1, 34.9, 0.329, 69.8}}},
+    {{{7.81, 2.47, 0.008, 4.65, 72.4, 14.4, 40.2, 0.319, 74.5},
+      {5.59, 4.18, 0.369, 11.5, 0.0, 11.5, 39.9, 0.117, 55.9}},
+     {{8.66, 1.42, 0.0, 4.33, 42.1, 10.9, 39.2, 0.568, 81.0},
+      {4.07, 6.30, 0.209, 7.94, 0.0, 8.39, 36.7, 0.316, 73.7}}},
+    {{{6.73, 2.94, 0.104, 7.74, 51.6, 15.3, 40.8, 0.250, 75.0},
+      {3.12, 7.32, 0.284, 11.8, 0.0, 10.2, 39.3, 0.069, 57.9}},
+     {{8.23, 0.59, 0.085, 6.61, 36.0, 11.7, 42.2, 0.517, 78.7},
+      {1.64, 7.18, 0.196, 9.28, 0.0, 9.73, 37.8, 0.335, 72.0}}},
 };
 
 // one(w) summed over the rounds of wgs workgroups, `at_once` at a time
