@@ -32,7 +32,7 @@ namespace {
 // float32 15.7 to 10.4 ms (16.4 clocks of a CU per step; the vector
 // instructions and the atomics take about 12 each, and either alone with the
 // loads 13 to 14); 3D 93x77x101 with 12 x 195, float16 tables, 1.89 to 1.12
-// ms; 2D 601x300 with 61 x 301, dynamic float32, RB = 8, 3.58 to 3.54 ms:
+// ms; 2D 601x300 with 61 x 301, dynamic float32, RB = 8, 3.58 to 3.51 ms:
 // bound by its loads (12 bytes per triplet through L1; without them 2.0 ms,
 // without the atomics 3.5 ms).
 constexpr int kSlotsMaxThreads = 1024;
@@ -55,11 +55,13 @@ template <int N> __device__ __forceinline__ float row_bcast(float v)
 // wait states of a vector instruction that wrote it.  The compiler sees to it
 // for the builtin but does not look into the instructions written here, and
 // may copy or reload their operands right before them: they wait themselves
-// (2D 601x300 dynamic float32 with 61 x 301 traces 3.49 ms with one wait per
-// tile ahead of all of them, 3.54 so; other shapes 0 to 1% more).
-#define KX_HALF2(OP)                                                                           \
-    "s_nop 1\n\t" OP "_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0x3\n\t" OP       \
-    "_dpp %0, %1, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xc"
+// (601x300 with 61 x 301 traces, float32: dynamic 3.50 ms with one wait per
+// tile ahead of all of them and 3.50 so, 3.54 with a wait for each of the
+// three pairs; kinematic, three waits a step, 2.29 and 2.32).
+#define KX_PAIR(OP, R, V, X, LO, HI)                                                           \
+    OP "_dpp " R ", " V ", " X " row_newbcast:" LO " row_mask:0xf bank_mask:0x3\n\t" OP          \
+       "_dpp " R ", " V ", " X " row_newbcast:" HI " row_mask:0xf bank_mask:0xc"
+#define KX_HALF2(OP) "s_nop 1\n\t" KX_PAIR(OP, "%0", "%1", "%2", "%3", "%4")
 template <int RB, int N> __device__ __forceinline__ float point_add(float v, float x)
 {
     if constexpr (RB == 16)
@@ -76,12 +78,22 @@ template <int RB, int N> __device__ __forceinline__ float point_mul(float v, flo
     asm(KX_HALF2("v_mul_f32") : "=&v"(r) : "v"(v), "v"(x), "n"(N), "n"(N + 8));
     return r;
 }
-template <int RB, int N> __device__ __forceinline__ float point_fma(float v, float x, float y)
+// T = ov + ox and w = pv px + qv qx, ov, pv and qv those of the point (the
+// three pairs share one wait: none writes what another broadcasts)
+template <int RB, int N>
+__device__ __forceinline__ void point_time_weight(float ov, float ox, float pv, float px, float qv,
+                                                  float qx, float &T, float &w)
 {
-    if constexpr (RB == 16)
-        return fmaf(row_bcast<N>(v), x, y);
-    asm(KX_HALF2("v_fmac_f32") : "+v"(y) : "v"(v), "v"(x), "n"(N), "n"(N + 8));
-    return y;
+    if constexpr (RB == 16) {
+        T = row_bcast<N>(ov) + ox;
+        w = fmaf(row_bcast<N>(qv), qx, row_bcast<N>(pv) * px);
+    } else {
+        asm("s_nop 1\n\t" KX_PAIR("v_add_f32", "%0", "%2", "%3", "%8", "%9") "\n\t"
+            KX_PAIR("v_mul_f32", "%1", "%4", "%5", "%8", "%9") "\n\t"
+            KX_PAIR("v_fmac_f32", "%1", "%6", "%7", "%8", "%9")
+            : "=&v"(T), "=&v"(w)
+            : "v"(ov), "v"(ox), "v"(pv), "v"(px), "v"(qv), "v"(qx), "n"(N), "n"(N + 8));
+    }
 }
 template <int RB, int N> __device__ __forceinline__ int point_sub(int v, int x)
 {
@@ -99,6 +111,7 @@ template <int RB, int N> __device__ __forceinline__ int point_value(int v)
     return __builtin_amdgcn_update_dpp(lo, v, 0x150 + (N & 7) + 8, 0xf, 0xc, false);
 }
 #undef KX_HALF2
+#undef KX_PAIR
 
 // A chunk of consecutive points' entries of one receiver.
 template <typename TT, typename RW, bool DYN> struct SlotChunk {
@@ -192,7 +205,11 @@ __device__ __forceinline__ void slot_point(const SlotChunk<TT, RW, DYN> &K, floa
 {
     constexpr int u = N % SlotChunkLen<TT>::v;
     // (broadcasts outside any branch: a lane switched off hands out nothing)
-    const float T = point_add<RB, N>(os, ld_off(&K.o.v[u]));
+    float T, w = 0.f, w1;
+    if constexpr (DYN)
+        point_time_weight<RB, N>(os, ld_off(&K.o.v[u]), mps, wv(K.p.v[u]), mqs, wv(K.q.v[u]), T, w);
+    else
+        T = point_add<RB, N>(os, ld_off(&K.o.v[u]));
     const int pz = DYN && GATE ? point_value<RB, N>(iz) : 0;
     float f;
     int k;
@@ -208,9 +225,7 @@ __device__ __forceinline__ void slot_point(const SlotChunk<TT, RW, DYN> &K, floa
             f -= 1.f;
         }
     }
-    float w = 0.f, w1;
     if constexpr (DYN) {
-        w = point_fma<RB, N>(mqs, wv(K.q.v[u]), point_mul<RB, N>(mps, wv(K.p.v[u])));
         w1 = w * f;
     } else {
         w1 = point_mul<RB, N>(mv, f);
