@@ -393,8 +393,8 @@ double slots_time(const kx_plan *p, const SlotsShape &g, int nh, int cus)
     return t;
 }
 
-// The shape with the smallest estimated time; the slots have to be 2% faster
-// than the kernels of 4, 2 and 1.  Where the pairs are no multiple of the
+// The shape with the smallest estimated time; a shape replaces a simpler one
+// where it is more than 1% faster.  Where the pairs are no multiple of the
 // workgroups that run at once, the last ones may be shared by several
 // workgroups, in work_bytes of scratch, whose sums a second launch adds (four
 // loads of a thread in flight: counts of parts that are no multiple of 4
@@ -410,11 +410,10 @@ SlotsShape pick_slots(const kx_plan *p, int nh, int64_t work_bytes, bool two_lau
         (p->rblock > 0 && p->rblock < 8))
         return best;
     const int cus = device_cus();
-    double best_t = p->rblock == 0 ? 0.98 * rows_time(p, nh, cus, two_launches) : 1e300;
+    double best_t = p->rblock == 0 ? rows_time(p, nh, cus, two_launches) : 1e300;
     auto consider = [&](SlotsShape g) {
-        const double t = nh > 0 && !g.fused
-                             ? 1.05 * (slots_time(p, g, 0, cus) + conv_time(p, nh, cus))
-                             : slots_time(p, g, nh, cus);
+        const double t = nh > 0 && !g.fused ? slots_time(p, g, 0, cus) + conv_time(p, nh, cus)
+                                            : slots_time(p, g, nh, cus);
         if (t < best_t * 0.99) {
             best_t = t;
             best = g;
